@@ -11,6 +11,7 @@
 //   gate_up  grouped GEMM over experts: x rows of the expert x W_gu[e] (+ bias), with
 //            the SwiGLU epilogue clamp(silu(gate), -limit, limit) * up fused in
 //   down     grouped GEMM over experts: h x W_down[e] (+ bias)
+//            (gate_up and down of up to 16 tokens: moe_few_kernel, else moe_stream_kernel)
 //   combine  y[t] = sum of w * y_e[t] over the token's experts in ascending expert
 //            order, the order of moe_forward's index_add (:171-189)
 //
@@ -173,6 +174,26 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
     return (int)(b[0] + b[1]);
 }
 
+// Logit (t, c): the nsplit slabs [T][E] summed in slab order, plus the bias when given.
+// The sum is one dependent chain, but its loads are not: eight slabs' loads are issued
+// together (one load per step waited for L2 each time: 15.6 us for one token's 64 slabs).
+__device__ __forceinline__ float slab_sum(const float *slabs, int nsplit, int64_t T, int E, int64_t t, int c,
+                                          const float *bias) {
+    const float *p = slabs + t * E + c;
+    const int64_t step = T * E;
+    const float b = bias ? bias[c] : 0.0f;
+    float v = p[0];
+    for (int s0 = 1; s0 < nsplit; s0 += 8) {
+        float q[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) q[j] = p[min(s0 + j, nsplit - 1) * step];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (s0 + j < nsplit) v += q[j];
+    }
+    return bias ? v + b : v;
+}
+
 // `logits` holds nsplit slabs [T][E] whose sum in slab order, plus `bias` when given,
 // are the logits (the router's K parts; nsplit = 1 and no bias: logits given)
 __global__ __launch_bounds__(256) void moe_route_kernel(const float *logits, int nsplit, const float *bias, int64_t T,
@@ -189,10 +210,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *logits, int
     for (int j = 0; j < 4; j++) {
         const int c = lane + 64 * j;
         if (c < E) {
-            float lv = logits[t * E + c];
-            for (int sp = 1; sp < nsplit; sp++) lv += logits[((int64_t)sp * T + t) * E + c];
-            if (bias) lv += bias[c];
-            v[j] = lv;
+            v[j] = slab_sum(logits, nsplit, T, E, t, c, bias);
         } else {
             v[j] = -INFINITY;
         }
@@ -345,9 +363,7 @@ __global__ __launch_bounds__(256) void moe_route_any_kernel(const float *logits,
     float mx = -INFINITY;
     int ninf = 0;
     for (int c = lane; c < E; c += 64) {
-        float lv = logits[t * E + c];
-        for (int sp = 1; sp < nsplit; sp++) lv += logits[((int64_t)sp * T + t) * E + c];
-        if (bias) lv += bias[c];
+        const float lv = slab_sum(logits, nsplit, T, E, t, c, bias);
         v[c] = lv;
         mx = fmaxf(mx, lv);
         ninf += lv == INFINITY;
@@ -723,10 +739,13 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const void *x, int64
     }
 }
 
-// K parts of the router: enough workgroups to spread the loads, at most 4 batches per wave
+// K parts of the router: enough workgroups to spread the loads, at most 4 batches per wave,
+// and no more parts than leave every wave two chunks (a few tokens' parts are all latency:
+// 23 parts instead of 64 at 2880 take the same time here and a third of the slab sum)
 inline int router_parts(int64_t T, int64_t H, int E) {
     const int64_t tiles = ((T + 15) / 16) * ((E + 15) / 16), nch = H / 16;
-    int64_t ks = std::max<int64_t>((256 + tiles - 1) / tiles, (nch + 4 * 4 * kRouterBatch - 1) / (4 * 4 * kRouterBatch));
+    int64_t ks = std::min<int64_t>((256 + tiles - 1) / tiles, (nch + 7) / 8);
+    ks = std::max<int64_t>(ks, (nch + 4 * 4 * kRouterBatch - 1) / (4 * 4 * kRouterBatch));
     return (int)std::min<int64_t>(std::min<int64_t>(ks, nch), 64);
 }
 
@@ -1129,9 +1148,295 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
     }
 }
 
+// ---------------------------------------------------------------------------------
+// expert GEMMs of a few tokens (decode): at most kMoeFewT tokens, bound by the weight
+// stream (13.2 MB per used expert of GPT-OSS: 53 MB, 7 to 10 us, for one token).
+// moe_stream_kernel's eight workgroups per expert would leave most CUs idle there, so here
+// an item is one column stream of one used expert (and up to kMoeFewRows of its rows; more
+// rows repeat the stream, from the caches), 360 items of each kernel for one token, and the
+// waves of a workgroup split its K.  Two workgroups per CU loop over the items.  A wave's
+// unit is a batch of NKB k-blocks: scales and its slice of the token rows go into LDS areas
+// of its own (no barrier), the codes into registers; a unit's loads are issued before the
+// previous one's math, across items too, so the stream does not stop for the conversion, the
+// sums' meeting in LDS and the epilogue.
+// Rows of the sorted buffers are the assignments themselves (row t * k + s), so there is
+// no permutation: a workgroup finds its experts in order of first appearance among the
+// assignments, by ballots over the routed experts.
+// The GPT-OSS layer (32 experts, top 4, 2880 x 2880) with its router: 1 token 107 -> 32 us,
+// 4 tokens 116 -> 59, 8 tokens 121 -> 91, 16 tokens 124 -> 112 (64 experts of 2880 x 1440,
+// top 8, 16 tokens: 163 -> 129); at 16 tokens most experts are in use and the two
+// organisations meet, so the rule (few, launch_moe) stops there.  At 8 tokens gate_up takes
+// 47 us of which its loads alone 24: the rest is the conversion (24 VALU per k-block and
+// column block) and the barrier per item.  One-shot workgroups without the loop: 136 us.
+// ---------------------------------------------------------------------------------
+constexpr int kMoeFewT = 16;        // tokens
+constexpr int kMoeFewAssign = 128;  // assignments: two per lane of the ballots
+constexpr int kMoeFewWaves = 8;
+constexpr int kMoeFewRows = 4;    // rows of an item
+constexpr int kMoeFewKb = 6;      // most k-blocks of a batch
+constexpr int kMoeFewGrid = 512;  // two workgroups per CU
+
+// XF: gate_up over f32 activations, staged as they are and split into bf16 hi + lo in registers
+template <bool GU, bool XF, int NKB>
+struct MoeFew {
+    static constexpr int P = GU && !XF ? 1 : 2;     // operand planes
+    static constexpr int NBW = GU ? 2 : 1;          // column blocks of a stream
+    static constexpr int SRC = GU ? 1 : 2;          // staged row sources (down: hi and lo)
+    static constexpr int RG = NKB * (XF ? 8 : 4);   // 16-byte granules of a staged row
+    static constexpr int WAVE = NBW * NKB * 32 + SRC * kMoeFewRows * RG * 16;  // a wave's staging bytes of a batch
+    static constexpr int RED = kMoeFewWaves * kMoeFewRows * NBW * 32;          // f32 of one reduction buffer
+    static constexpr int EPI = NBW * 128 + kMoeFewRows * 4;  // an item's bias columns and rows
+    static constexpr int LDS = 2 * kMoeFewWaves * WAVE + 2 * RED * 4 + 3 * EPI;
+    static_assert(2 * (LDS + 1024) <= 160 * 1024, "two workgroups per CU");
+    static_assert(2 * NKB * NBW + NBW + 1 < 64, "vmcnt range");
+};
+
+template <bool GU, bool XF, int NKB>
+__global__ __launch_bounds__(kMoeFewWaves * 64, 4) void moe_few_kernel(MoeDev d, MoeScratch sc, MoeRun run,
+                                                                       const float *xf) {
+    using F = MoeFew<GU, XF, NKB>;
+    constexpr int P = F::P, NBW = F::NBW, SRC = F::SRC, RG = F::RG, C = NBW * 32;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __shared__ int32_t rows[kMoeFewWaves][kMoeFewT];  // the expert's assignments, a copy per wave
+    const int64_t H = d.H, I = d.I;
+    const int KB = (int)((GU ? H : I) / 32), NB = (int)(GU ? 2 * I / 32 : H / 32);
+    const int S = moe_streams(GU, H, I);
+    const int tid = threadIdx.x, lane = tid & 63, nw = (int)blockDim.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = lane >> 4, l16 = lane & 15;
+    const int k0 = wv * KB / nw, k1 = (wv + 1) * KB / nw;     // this wave's k-blocks
+    const int nbatch = ((KB + nw - 1) / nw + NKB - 1) / NKB;  // the same in every wave
+    unsigned char *stage = smem + 2 * wv * F::WAVE;           // two batches: [scales][rows]
+    float *red = reinterpret_cast<float *>(smem + 2 * kMoeFewWaves * F::WAVE);
+    unsigned char *epi = smem + 2 * kMoeFewWaves * F::WAVE + 2 * F::RED * 4;
+
+    // the assignments' experts, two per lane
+    const int A = (int)run.A;
+    const uint32_t none = 0xFFFFFFFFu;
+    const uint32_t t0 = lane < A ? run.ti[lane] : none, t1 = lane + 64 < A ? run.ti[lane + 64] : none;
+    uint64_t left0 = __ballot(t0 != none), left1 = __ballot(t1 != none);
+    // the unit of work to issue next: batch bt of K of rows g0 .. g0 + 3 (below ne) of stream
+    // st of the slot-th distinct expert e; eb its item's epilogue buffer
+    int slot = -1, ne = 0, st = (int)blockIdx.x, g0 = 0, bt = 0, eb = 0;
+    int64_t e = 0;
+    // steps to the slot of stream st (S streams each): false when there is none
+    auto seek = [&]() {
+        while (slot < 0 || st >= S) {
+            if (slot >= 0) st -= S;
+            if ((left0 | left1) == 0) return false;
+            slot++;
+            const uint32_t ex = left0 ? (uint32_t)__builtin_amdgcn_readlane((int)t0, __builtin_ctzll(left0))
+                                      : (uint32_t)__builtin_amdgcn_readlane((int)t1, __builtin_ctzll(left1));
+            const uint64_t m0 = __ballot(t0 == ex), m1 = __ballot(t1 == ex);
+            left0 &= ~m0;
+            left1 &= ~m1;
+            e = ex;
+            ne = __popcll(m0) + __popcll(m1);  // <= tokens <= 16
+            const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+            if ((m0 >> lane) & 1) rows[wv][__popcll(m0 & lt)] = lane;
+            if ((m1 >> lane) & 1) rows[wv][__popcll(m0) + __popcll(m1 & lt)] = lane + 64;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        return true;
+    };
+    auto advance = [&]() {
+        if (++bt < nbatch) return true;
+        bt = 0;
+        eb = eb == 2 ? 0 : eb + 1;
+        g0 += kMoeFewRows;
+        if (g0 < ne) return true;
+        g0 = 0;
+        st += (int)gridDim.x;
+        return seek();
+    };
+
+    // buffer resources: scalar bases, 32-bit lane offsets (the rows span at most 16 x 32768
+    // f32, the h planes 2 x 128 x 32768 bf16; offsets past an end read zeros, of k-blocks
+    // that are not used)
+    const int row_bytes = (int)(GU ? H : I) * (XF ? 4 : 2), plane_bytes = (int)(run.A * I * 2);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<void *>(GU ? (XF ? (const void *)xf : (const void *)run.xa[0]) : (const void *)sc.hb), 0,
+        GU ? (int)run.T * row_bytes : 2 * plane_bytes, 0x00020000);
+    u32x2 wq[2][NKB][NBW];
+    auto issue = [&](int slot2) {
+        const int nr = min(ne - g0, kMoeFewRows), kb = k0 + bt * NKB;
+        unsigned char *scl = stage + slot2 * F::WAVE, *xl = scl + NBW * NKB * 32;
+        // the item's bias columns and assignments, for its epilogue (LDS, not registers held
+        // over the item)
+        if (wv == 0 && bt == 0) {
+            unsigned char *ep = epi + eb * F::EPI;
+            if (lane < kMoeFewRows) reinterpret_cast<int32_t *>(ep + NBW * 128)[lane] = rows[0][g0 + min(lane, nr - 1)];
+            const float *bp = GU ? d.gu_b + e * 2 * I : d.dn_b + e * H;
+            const __amdgpu_buffer_rsrc_t rb =
+                __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(bp), 0, NB * 128, 0x00020000);
+            if (lane < 8)
+#pragma unroll
+                for (int b = 0; b < NBW; b++) moe_copy16_lds(rb, ep + b * 128, 16 * lane, (b * NB / 2 + st) * 128);
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the staging area
+        __amdgpu_buffer_rsrc_t rq[NBW], rs[NBW];
+#pragma unroll
+        for (int b = 0; b < NBW; b++) {
+            const int64_t nb = e * NB + (b == 0 ? st : NB / 2 + st);
+            rq[b] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>((GU ? d.gu_q : d.dn_q) + nb * KB * 512), 0,
+                                                      KB * 512, 0x00020000);
+            rs[b] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>((GU ? d.gu_s : d.dn_s) + nb * KB * 32), 0,
+                                                      KB * 32, 0x00020000);
+        }
+        if (lane < NKB * 2)
+#pragma unroll
+            for (int b = 0; b < NBW; b++) moe_copy16_lds(rs[b], scl + b * NKB * 32, 16 * lane, kb * 32);
+        // staged row r's granule g sits at slot moe_slot(g, r) of the row; the rows (down:
+        // of the hi plane, then of the lo plane) pack into 64-granule copies
+#pragma unroll
+        for (int i0 = 0; i0 < SRC * kMoeFewRows * RG; i0 += 64) {
+            const int i = i0 + lane;
+            if (i < SRC * nr * RG) {
+                int r = i / RG;
+                const int lo = SRC == 2 && r >= nr;
+                r -= lo ? nr : 0;
+                const int a = rows[wv][g0 + r], g = moe_slot(i % RG, r);
+                moe_copy16_lds(ra, xl + i0 * 16, (uint32_t)((GU ? a / run.k : a) * row_bytes + lo * plane_bytes + 16 * g),
+                               kb * (XF ? 128 : 64));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the codes last: the waits below count them
+#pragma unroll
+        for (int j = 0; j < NKB; j++)
+#pragma unroll
+            for (int b = 0; b < NBW; b++)
+                // past the wave's range: a repeat, not used; cache policy 2: non-temporal
+                wq[slot2][j][b] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                                                rq[b], 8 * lane, max(min(kb + j, k1 - 1), 0) * 512, 2));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    if (!seek()) return;  // workgroup-uniform, as every branch below on the unit
+    issue(0);
+    floatx4 acc[NBW][2];
+#pragma unroll
+    for (int b = 0; b < NBW; b++) acc[b][0] = acc[b][1] = zero4();
+    int buf = 0;  // reduction buffer
+    // computes the unit in slot U while the next one's loads (slot 1 - U) are in flight; false
+    // after the last
+    auto step = [&](auto u_c) {
+        constexpr int U = decltype(u_c)::value;
+        const int nr = min(ne - g0, kMoeFewRows), kb = k0 + bt * NKB, ist = st, ieb = eb;
+        const bool item_done = bt + 1 == nbatch;
+        const bool more = advance();
+        if (more) issue(1 - U);
+        // this lane's two operand sources: bf16 rows, granule 4j + p of the plane's row; f32
+        // rows, granules 8j + 2p and 8j + 2p + 1 (the slot's xor stays inside aligned groups
+        // of 4); rows past the item's repeat its last one (results not used)
+        const int rr = min(l16, nr - 1);
+        const unsigned char *scl = stage + U * F::WAVE, *xl = scl + NBW * NKB * 32;
+        const unsigned char *xr[2];
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+            xr[q] = xl + ((XF ? rr : (q < P ? q : 0) * nr + rr) * RG + moe_slot(XF ? 2 * p + q : p, rr)) * 16;
+        // this unit's staged bytes: at least its codes, and the next unit's scales, one copy
+        // and codes were issued after them
+        __builtin_amdgcn_sched_barrier(0);
+        if (more)
+            wait_vmcnt<2 * NKB * NBW + NBW + 1>();
+        else
+            wait_vmcnt<NKB * NBW>();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NKB; j++) {
+            if (kb + j < k1) {  // wave-uniform
+                u32x4 av[P];
+                if constexpr (XF) {
+                    const u32x4 f[2] = {*reinterpret_cast<const u32x4 *>(xr[0] + j * 128),
+                                        *reinterpret_cast<const u32x4 *>(xr[1] + j * 128)};
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const uint32_t f0 = f[q >> 1][2 * (q & 1)], f1 = f[q >> 1][2 * (q & 1) + 1];
+                        const uint32_t h0 = bf16_rne(__uint_as_float(f0)), h1 = bf16_rne(__uint_as_float(f1));
+                        av[0][q] = h0 | (h1 << 16);
+                        av[1][q] = (uint32_t)bf16_rne(__uint_as_float(f0) - bf16_to_f32(h0)) |
+                                   ((uint32_t)bf16_rne(__uint_as_float(f1) - bf16_to_f32(h1)) << 16);
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < P; q++) av[q] = *reinterpret_cast<const u32x4 *>(xr[q] + j * 64);
+                }
+#pragma unroll
+                for (int b = 0; b < NBW; b++) {
+                    const u32x2 sw = *reinterpret_cast<const u32x2 *>(scl + (b * NKB + j) * 32 + 8 * p);
+                    uint32_t r[8];
+                    fp4_rows(wq[U][j][b], sw, r);
+                    u32x4 be, bo;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        bo[q] = __builtin_amdgcn_perm(r[2 * q + 1], r[2 * q], 0x05040100u);  // column 2c + 1
+                        be[q] = __builtin_amdgcn_perm(r[2 * q + 1], r[2 * q], 0x07060302u);  // column 2c
+                    }
+#pragma unroll
+                    for (int q = 0; q < P; q++) {
+                        acc[b][0] = mfma16x16x32_bf16(av[q], be, acc[b][0]);
+                        acc[b][1] = mfma16x16x32_bf16(av[q], bo, acc[b][1]);
+                    }
+                }
+            }
+        }
+        if (item_done) {
+            // the waves' sums: [wave][row][column] in alternating buffers (a buffer is written
+            // again after the other one's barrier, past which its readers have gone; an
+            // item's epilogue data, written up to two units ahead, has three)
+            float *rb = red + buf * F::RED;
+            if (p == 0) {  // rows 0 .. 3 of the tile
+#pragma unroll
+                for (int i = 0; i < kMoeFewRows; i++)
+#pragma unroll
+                    for (int b = 0; b < NBW; b++)
+                        *reinterpret_cast<float2 *>(rb + (wv * kMoeFewRows + i) * C + b * 32 + 2 * l16) =
+                            float2{acc[b][0][i], acc[b][1][i]};
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) only: the next unit's loads stay in flight
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            if (tid < nr * 32) {
+                const int ec = tid & 31, er = tid >> 5;  // column of the stream, row of the item
+                const unsigned char *ep = epi + ieb * F::EPI;
+                const int64_t col = (int64_t)ist * 32 + ec, ar = reinterpret_cast<const int32_t *>(ep + NBW * 128)[er];
+                float s[NBW];
+#pragma unroll
+                for (int b = 0; b < NBW; b++) s[b] = 0.0f;
+                for (int w = 0; w < nw; w++)
+#pragma unroll
+                    for (int b = 0; b < NBW; b++) s[b] += rb[(w * kMoeFewRows + er) * C + b * 32 + ec];
+#pragma unroll
+                for (int b = 0; b < NBW; b++) s[b] += reinterpret_cast<const float *>(ep + b * 128)[ec];
+                if constexpr (GU) {
+                    const float gt = s[0], up = s[NBW - 1];
+                    float sg = gt / (1.0f + expf(-gt));  // silu, clamped to +-limit, as moe_stream_kernel
+                    sg = sg < -run.limit ? -run.limit : (sg > run.limit ? run.limit : sg);
+                    const float h = sg * up;
+                    const uint32_t bh = bf16_rne(h);
+                    sc.hb[ar * I + col] = (uint16_t)bh;
+                    sc.hb[(run.A + ar) * I + col] = bf16_rne(h - bf16_to_f32(bh));
+                    if (col == 0) sc.pos[ar] = (int32_t)ar;  // for the combine: an assignment's row is itself
+                } else {
+                    sc.yb[ar * H + col] = s[0];
+                }
+            }
+            buf ^= 1;
+#pragma unroll
+            for (int b = 0; b < NBW; b++) acc[b][0] = acc[b][1] = zero4();
+        }
+        return more;
+    };
+    while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
+    }
+}
+
 // y[t] = ((0 + w_a * y_a) + w_b * y_b) + ... over the token's experts a < b < ...
 // A NaN or infinite output sets *status (when given) to NNQ_ERR_NON_FINITE, the
 // check_output_finite of moe_forward (crates/nn-core/src/layers/nan_check.rs:113-140).
+// grid.y workgroups share a token's columns (a few tokens alone would leave the chip idle).
 template <int k, bool V4>
 __global__ __launch_bounds__(256) void moe_combine_kernel(MoeScratch sc, int64_t H, float *y, int32_t *status) {
     const int64_t t = blockIdx.x;
@@ -1165,7 +1470,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeScratch sc, int64_t
         // per-element arithmetic on 16-byte loads and stores
         const int64_t H4 = H / 4;
 #pragma unroll 3
-        for (int64_t c = threadIdx.x; c < H4; c += 256) {
+        for (int64_t c = (int64_t)blockIdx.y * 256 + threadIdx.x; c < H4; c += 256 * (int64_t)gridDim.y) {
             floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int s = 0; s < k; s++) {
@@ -1178,7 +1483,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeScratch sc, int64_t
             for (int i = 0; i < 4; i++) bad |= !(fabsf(acc[i]) <= 3.402823466e38f);
         }
     } else {
-        for (int64_t c = threadIdx.x; c < H; c += 256) {
+        for (int64_t c = (int64_t)blockIdx.y * 256 + threadIdx.x; c < H; c += 256 * (int64_t)gridDim.y) {
             float acc = 0.0f;
 #pragma unroll
             for (int s = 0; s < k; s++) acc = acc + sc.yb[(int64_t)ps[s] * H + c] * ws[s];
@@ -1329,6 +1634,34 @@ static int launch_stream(const MoeDev &d, const MoeScratch &sc, const MoeRun &ru
     return launch_stream_t<P, GU, 1, false>(d, sc, run, st, moe_lds<P, GU, 1, false>(KB));
 }
 
+template <bool GU, bool XF, int NKB>
+static int launch_few_t(const MoeDev &d, const MoeScratch &sc, const MoeRun &run, const float *xf, int64_t nw,
+                        hipStream_t st) {
+    constexpr int LDS = MoeFew<GU, XF, NKB>::LDS;
+    static bool attr_set = false;  // idempotent attribute write; races only repeat it
+    if (!attr_set) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_few_kernel<GU, XF, NKB>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        if (e != hipSuccess) return (int)e;
+        attr_set = true;
+    }
+    const int64_t items = std::min<int64_t>(d.E, run.A) * moe_streams(GU, d.H, d.I);
+    hipLaunchKernelGGL((moe_few_kernel<GU, XF, NKB>), dim3((unsigned)std::min<int64_t>(items, kMoeFewGrid)),
+                       dim3((unsigned)nw * 64), LDS, st, d, sc, run, xf);
+    return (int)hipGetLastError();
+}
+
+template <bool GU, bool XF>
+static int launch_few(const MoeDev &d, const MoeScratch &sc, const MoeRun &run, const float *xf, hipStream_t st) {
+    // the fewest waves that keep the longest wave's share of K, at least the two whose threads
+    // write an item's rows; batches of 6 k-blocks past a share of 4 (90: 8 waves of 11 or 12)
+    const int64_t KB = (GU ? d.H : d.I) / 32;
+    const int64_t per = (KB + kMoeFewWaves - 1) / kMoeFewWaves, nw = std::max<int64_t>((KB + per - 1) / per, 2);
+    if (per <= 2) return launch_few_t<GU, XF, 2>(d, sc, run, xf, nw, st);
+    if (per <= 4) return launch_few_t<GU, XF, 4>(d, sc, run, xf, nw, st);
+    return launch_few_t<GU, XF, kMoeFewKb>(d, sc, run, xf, nw, st);
+}
+
 int launch_moe(const MoeDev &d, const void *x, int x_bf16, int64_t T, const float *logits, int nsplit,
                const float *bias, int k, float limit, float *y, uint32_t *topk_idx, float *topk_w, int32_t *status,
                void *scratch, void *stream) {
@@ -1342,6 +1675,7 @@ int launch_moe(const MoeDev &d, const void *x, int x_bf16, int64_t T, const floa
     run.T = T;
     run.k = k;
     run.perm = T <= kMoeInPermT ? 1 : 0;
+    const bool few = T <= kMoeFewT && run.A <= kMoeFewAssign;
     if (d.E <= 256)
         hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, logits, nsplit, bias, T,
                            (int)d.E, k, sc.ti, sc.tw, topk_idx, topk_w);
@@ -1362,31 +1696,33 @@ int launch_moe(const MoeDev &d, const void *x, int x_bf16, int64_t T, const floa
                            sc.off, sc.stok, sc.pos);
         break;
     }
-    if (x_bf16) {
-        run.xa[0] = reinterpret_cast<const uint16_t *>(x);
-        run.xa[1] = nullptr;
+    run.xa[0] = x_bf16 ? reinterpret_cast<const uint16_t *>(x) : sc.xb;
+    run.xa[1] = x_bf16 ? nullptr : sc.xb + T * d.H;
+    if (few) {
+        const float *xf = reinterpret_cast<const float *>(x);
+        e = x_bf16 ? launch_few<true, false>(d, sc, run, nullptr, st) : launch_few<true, true>(d, sc, run, xf, st);
+        if (!e) e = launch_few<false, false>(d, sc, run, nullptr, st);
     } else {
-        const int64_t n = T * d.H;
-        hipLaunchKernelGGL(moe_split_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                           reinterpret_cast<const float *>(x), n, sc.xb);
-        run.xa[0] = sc.xb;
-        run.xa[1] = sc.xb + n;
+        if (!x_bf16) {
+            const int64_t n = T * d.H;
+            hipLaunchKernelGGL(moe_split_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                               reinterpret_cast<const float *>(x), n, sc.xb);
+        }
+        e = x_bf16 ? launch_stream<1, true>(d, sc, run, st) : launch_stream<2, true>(d, sc, run, st);
+        if (!e) e = launch_stream<2, false>(d, sc, run, st);
     }
-    if (x_bf16)
-        e = launch_stream<1, true>(d, sc, run, st);
-    else
-        e = launch_stream<2, true>(d, sc, run, st);
-    if (e) return e;
-    e = launch_stream<2, false>(d, sc, run, st);
     if (e) return e;
     const bool v4 = d.H % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+    // below one workgroup per CU a token's columns are shared out, 256 threads' worth each
+    const int64_t cparts = (d.H / (v4 ? 4 : 1) + 255) / 256;
+    const dim3 cgrid((unsigned)T, (unsigned)(T < 256 ? cparts : 1));
     switch (k) {
 #define NNQ_COMB(K)                                                                                         \
     case K:                                                                                                 \
         if (v4)                                                                                             \
-            hipLaunchKernelGGL((moe_combine_kernel<K, true>), dim3((unsigned)T), dim3(256), 0, st, sc, d.H, y, status); \
+            hipLaunchKernelGGL((moe_combine_kernel<K, true>), cgrid, dim3(256), 0, st, sc, d.H, y, status); \
         else                                                                                                \
-            hipLaunchKernelGGL((moe_combine_kernel<K, false>), dim3((unsigned)T), dim3(256), 0, st, sc, d.H, y, status); \
+            hipLaunchKernelGGL((moe_combine_kernel<K, false>), cgrid, dim3(256), 0, st, sc, d.H, y, status); \
         break;
         NNQ_COMB(1) NNQ_COMB(2) NNQ_COMB(3) NNQ_COMB(4) NNQ_COMB(5) NNQ_COMB(6) NNQ_COMB(7) NNQ_COMB(8)
 #undef NNQ_COMB
