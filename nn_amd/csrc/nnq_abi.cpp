@@ -462,8 +462,8 @@ static int check_linear(const nnq_weight *w, const void *x, nnq_dtype xd, int64_
 
 }  // extern "C"
 
-// One validated linear call: the MFMA GEMM (gemm_batch) or GEMV passes of up to
-// 8 tokens.  GEMV-only options: x_swiglu (x holds gate | up rows of 2k f32, the input
+// One validated linear call: the few-row GEMM (few_batch), the MFMA GEMM (gemm_batch) or GEMV
+// passes of up to 4 tokens.  GEMV-only options: x_swiglu (x holds gate | up rows of 2k f32, the input
 // is silu(gate) * up; m <= 2 so one pass) and a status (mode 1 clears it in the
 // first pass, mode 2 flags non-finite outputs in every pass).
 static GemmArgs gemm_args(const nnq_weight *w, const void *x, nnq_dtype x_dtype, int64_t m, const float *bias, void *y,
@@ -487,18 +487,32 @@ static GemmArgs gemm_args(const nnq_weight *w, const void *x, nnq_dtype x_dtype,
     return g;
 }
 
-// scratch a linear call of m tokens needs (the prefill GEMM's staging and split-K slabs)
-// MFMA GEMM or GEMV passes (of up to 8 tokens for Q8_0, 4 otherwise), by the measured
-// crossover on MI355X: Q4_K from 3 tokens with bf16 activations (the one-launch thin
-// GEMM: 3 and 4 tokens at 12288x4096 in 8.8 / 8.9 us against 10.3 / 10.5 as a GEMV pass,
-// level at 4096x12288; 2 tokens: 8.7 against 7.7) and from 9 with f32 ones (23.6 against
-// 28.4 at 8), Q6_K from 9 (8 tokens at 4096x12288: two batched passes 27 us, GEMM 36.8), Q8_0
-// from 9 with bf16 activations and from 17 with f32 ones (8 tokens in one batched GEMV
-// pass: 7.9 us at 4096x4096, 17.9 at 4096x12288; 9 f32 tokens as GEMM: 20.9 and 39.2 us)
+// The path of a linear call of m tokens, by measured crossovers on MI355X (us, x f32 / bf16):
+//  - 1 and 2 tokens: one decode-GEMV pass;
+//  - 3 to 16: the few-row GEMM (few_batch), which reads the weight once, from 5 tokens on
+//    (Q8_0 4096x4096, 12 tokens: 14.3 / 17.0 as passes / GEMM, 12.8 / 7.5 here; Q6_K
+//    12288x4096, 8 tokens: 26.8 / 26.3 as two passes, 14.0 / 12.1).  Below that a GEMV pass of
+//    4 tokens has the shorter prologue (Q6_K 4096x4096: 6.2 against 8.4 / 7.4), except over
+//    many tiles per CU (4 tokens, Q6_K: 24576 rows 23.8 against 20.3, 60000 rows 56 against 42;
+//    Q8_0: 24576 rows level, 60000 rows 46.6 against 43.4).  Q4_K with f32 x takes it from 7
+//    tokens (4096x4096: 5 and 6 as two passes 8.6 and 9.0 against 9.1 and 9.3; 8: 10.5 against
+//    9.6), from 5 with two tiles per CU (24576 rows: 30.0 against 19.3) or K over 8192 (6
+//    tokens at 4096x12288: 19.0 against 17.2).  Q4_K with bf16 x keeps the thin GEMM, which
+//    stages nothing, up to that many tiles (16 tokens: 12288x4096 10.0 against 13.0, 24576
+//    rows 18.8 against 19.5, 60000 rows 45.2 against 37.6);
+//  - other counts: the MFMA GEMM.
+static bool few_batch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
+    const Layout &L = w->L;
+    if (m < 3 || m > 16 || L.k > ((int64_t)1 << 24) || L.ntile >= ((int64_t)1 << 31)) return false;
+    if (L.ntile >= 2048) return true;  // eight tiles per CU
+    if (L.fmt != NNQ_FMT_Q4_K) return m > 4;
+    if (x_dtype == NNQ_BF16) return false;
+    return m > 6 || (m > 4 && (L.ntile >= 512 || L.k > 8192));
+}
+
 static bool gemm_batch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
-    if (w->L.fmt == NNQ_FMT_Q4_K) return m > (x_dtype == NNQ_BF16 ? 2 : 8);
-    if (w->L.fmt == NNQ_FMT_Q6_K) return m > 8;
-    return m > (x_dtype == NNQ_BF16 ? 8 : 16);
+    if (few_batch(w, m, x_dtype)) return false;
+    return m > (w->L.fmt == NNQ_FMT_Q4_K ? (x_dtype == NNQ_BF16 ? 2 : 6) : 4);
 }
 
 // the prefill GEMM's scratch for m tokens run in launches of gemm_chunk_rows rows (the
@@ -510,7 +524,14 @@ static size_t gemm_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtyp
     return b;
 }
 
+// (a few-row call's launches are alike in the rows they take, so the first one's scratch does)
+static size_t few_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
+    const int64_t rows = std::min<int64_t>(m, gemm_few_rows(w->L.fmt));
+    return gemm_few_scratch_bytes(gemm_args(w, nullptr, x_dtype, rows, nullptr, nullptr, NNQ_F32), w->L.fmt);
+}
+
 static size_t linear_scratch_bytes(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
+    if (few_batch(w, m, x_dtype)) return few_call_scratch(w, m, x_dtype);
     if (!gemm_batch(w, m, x_dtype)) return 0;
     return gemm_call_scratch(w, m, x_dtype);
 }
@@ -545,9 +566,26 @@ static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype
         }
         return NNQ_OK;
     }
-    // tokens per GEMV pass: Q4_K and Q6_K up to 4 (their decode kernels with four token
-    // rows), Q8_0 up to 8 (its batched kernel)
-    const int64_t mmax = L.fmt == NNQ_FMT_Q8_0 ? 8 : 4;
+    if (!x_swiglu && !status && few_batch(w, m, x_dtype)) {
+        const int64_t mc = gemm_few_rows(L.fmt);
+        Scratch s;
+        void *scr = ext_scratch;
+        const size_t need = few_call_scratch(w, m, x_dtype);
+        if (!scr && need) {
+            HIP_TRY(s.alloc(need, (hipStream_t)stream), "scratch alloc");
+            scr = s.p;
+        }
+        for (int64_t m0 = 0; m0 < m; m0 += mc) {
+            GemmArgs g = gemm_args(w, (const uint8_t *)x + (size_t)m0 * k * xe, x_dtype, std::min(mc, m - m0), bias,
+                                   (uint8_t *)y + (size_t)m0 * L.n * ye, y_dtype);
+            g.scratch = scr;
+            int e = launch_gemm_few(g, L.fmt, stream);
+            if (e) return hip_fail((hipError_t)e, "gemm launch");
+        }
+        return NNQ_OK;
+    }
+    // tokens per GEMV pass: up to 4 (the decode kernels with four token rows)
+    const int64_t mmax = 4;
     const int64_t xrow = x_swiglu ? 2 * k : k;
     for (int64_t m0 = 0; m0 < m; m0 += mmax) {
         GemvArgs a{};

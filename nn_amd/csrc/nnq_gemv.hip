@@ -1101,9 +1101,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_decode_kernel(const uint8
 }
 
 // ---------------------------------------------------------------------------------
-// Q8_0 batched decode (3 <= m <= 8; MT = 4 or 8 token rows, the rows past m zero):
-// gemv_q80_decode_kernel's unit math with every A row in use (rows 2t + part), so lane
-// group g holds tokens 2g and 2g + 1.  The block statistics of every token go through a
+// Q8_0 batched decode (3 <= m <= 4; the rows of MT = 4 tokens, those past m zero):
+// gemv_q80_decode_kernel's unit math with A rows 2t + part, so lane group g holds tokens 2g
+// and 2g + 1 (more tokens: gemm_few_kernel).  The block statistics of every token go through a
 // per-wave LDS table (8 powers of two and 8 sums per token) that each lane group reads
 // for its two tokens with broadcast 16-byte reads.  One unit per wave and pass.
 // ---------------------------------------------------------------------------------
@@ -1929,29 +1929,24 @@ static int launch_q80_decode_t(const GemvArgs &a, void *stream) {
     if (a.x_swiglu) return launch_q80_decode_x<WAVES, UPW, 2>(a, stream);
     return a.x_bf16 ? launch_q80_decode_x<WAVES, UPW, 1>(a, stream) : launch_q80_decode_x<WAVES, UPW, 0>(a, stream);
 }
-template <int WAVES, int MT>
+template <int WAVES>
 static int launch_q80_batch_t(const GemvArgs &a, void *stream) {
     if (a.x_swiglu)
-        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 2, MT>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
+        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 2, 4>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
                            (hipStream_t)stream, a);
     else if (a.x_bf16)
-        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 1, MT>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
+        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 1, 4>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
                            (hipStream_t)stream, a);
     else
-        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 0, MT>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
+        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 0, 4>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
                            (hipStream_t)stream, a);
     return (int)hipGetLastError();
 }
-// Q8_0 batches of 3-8 tokens: 4 or 8 token rows, waves of one unit per pass: 16 when
-// the grid has at most two tiles per CU and K is over 8 units, else 8 (4 for K of up
-// to 4 units).  4096x4096, 8 tokens: 7.9 us (12.5 in the block GEMV form).
+// Q8_0 batches of 3-4 tokens: 4 token rows, waves of one unit per pass: 16 when the grid has
+// at most two tiles per CU and K is over 8 units, else 8 (4 for K of up to 4 units).
 static int launch_q80_batch(const GemvArgs &a, int64_t units, void *stream) {
-    const bool w16 = a.ntile <= 512 && units > 8;
-    if (a.m <= 4)
-        return units <= 4 ? launch_q80_batch_t<4, 4>(a, stream)
-                          : (w16 ? launch_q80_batch_t<16, 4>(a, stream) : launch_q80_batch_t<8, 4>(a, stream));
-    return units <= 4 ? launch_q80_batch_t<4, 8>(a, stream)
-                      : (w16 ? launch_q80_batch_t<16, 8>(a, stream) : launch_q80_batch_t<8, 8>(a, stream));
+    if (units <= 4) return launch_q80_batch_t<4>(a, stream);
+    return a.ntile <= 512 && units > 8 ? launch_q80_batch_t<16>(a, stream) : launch_q80_batch_t<8>(a, stream);
 }
 
 // Q8_0 decode shapes: one wave per unit up to 16 units, then 16 waves of up to

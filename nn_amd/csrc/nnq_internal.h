@@ -148,6 +148,12 @@ int launch_gemm_q4k(const GemmArgs &a, void *stream);
 // the shape (R, W: tiles per workgroup and waves), and its launch; no scratch
 int gemm_thin_plan(const GemmArgs &a, int *R, int *W);
 int launch_gemm_thin(const GemmArgs &a, void *stream);
+// one-launch GEMM over a few rows, the weight read once (nnq_gemm_few.hip): the rows of a
+// launch, its scratch (the K parts' slabs; 0 up to K = 4096), and the launch (a.m up to the
+// rows; a.x 16-byte aligned)
+int gemm_few_rows(int fmt);
+size_t gemm_few_scratch_bytes(const GemmArgs &a, int fmt);
+int launch_gemm_few(const GemmArgs &a, int fmt, void *stream);
 // Q8_0 / Q6_K prefill GEMM (M > 8): the activation staging below, then one kernel
 int launch_gemm_blk(const GemmArgs &a, void *stream);
 // its K split (and tile height and width, when bm / bn are given)

@@ -1395,9 +1395,11 @@ __global__ __launch_bounds__(kMoeFewWaves * 64, 4) void moe_few_kernel(MoeDev d,
                         *reinterpret_cast<float2 *>(rb + (wv * kMoeFewRows + i) * C + b * 32 + 2 * l16) =
                             float2{acc[b][0][i], acc[b][1][i]};
             }
+            asm volatile("" ::: "memory");
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0) only: the next unit's loads stay in flight
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
             if (tid < nr * 32) {
                 const int ec = tid & 31, er = tid >> 5;  // column of the stream, row of the item
                 const unsigned char *ep = epi + ieb * F::EPI;
