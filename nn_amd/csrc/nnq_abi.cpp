@@ -536,12 +536,20 @@ static size_t linear_scratch_bytes(const nnq_weight *w, int64_t m, nnq_dtype x_d
     return gemm_call_scratch(w, m, x_dtype);
 }
 
+// whether a prefill of m tokens can write h = silu(gate) * up from the gate | up GEMM: Q4_K, one
+// launch (the rows of y differ from the chunks' otherwise), the wide kernel without a K split
+static bool prefill_swiglu(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
+    return w->L.fmt == NNQ_FMT_Q4_K && m > 2 && gemm_batch(w, m, x_dtype) && gemm_chunk_rows(m, w->L.k) == m &&
+           gemm_wide_swiglu(gemm_args(w, nullptr, x_dtype, m, nullptr, nullptr, NNQ_F32));
+}
+
 static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype, int64_t m, const float *bias,
                            void *y, nnq_dtype y_dtype, void *stream, int x_swiglu = 0, int32_t *status = nullptr,
                            int status_mode = 0, void *ext_scratch = nullptr, int swiglu_out = 0) {
     if (m == 0) return NNQ_OK;
-    if (swiglu_out && (w->L.fmt != NNQ_FMT_Q4_K || m > 2 || x_swiglu || bias || w->L.n % 16))
-        return fail(NNQ_ERR_INVALID_ARGUMENT, "SwiGLU epilogue needs a Q4_K decode GEMV over whole tiles");
+    if (swiglu_out && (w->L.fmt != NNQ_FMT_Q4_K || (m > 2 && !prefill_swiglu(w, m, x_dtype)) || x_swiglu || bias ||
+                       w->L.n % 16))
+        return fail(NNQ_ERR_INVALID_ARGUMENT, "SwiGLU epilogue needs a Q4_K decode GEMV or wide GEMM over whole tiles");
     const Layout &L = w->L;
     const int64_t k = L.k;
     const size_t xe = x_dtype == NNQ_BF16 ? 2 : 4, ye = y_dtype == NNQ_BF16 ? 2 : 4;
@@ -561,6 +569,8 @@ static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype
             GemmArgs g = gemm_args(w, (const uint8_t *)x + (size_t)m0 * k * xe, x_dtype, rows, bias,
                                    (uint8_t *)y + (size_t)m0 * L.n * ye, y_dtype);
             g.scratch = scr;
+            g.swiglu_out = swiglu_out;
+            g.status = swiglu_out ? status : nullptr;
             int e = g.blk ? launch_gemm_blk(g, stream) : launch_gemm_q4k(g, stream);
             if (e) return hip_fail((hipError_t)e, "gemm launch");
         }
@@ -914,13 +924,14 @@ static int mlp_run(const nnq_mlp *p, const void *x, nnq_dtype x_dtype, int64_t m
     const int64_t I = p->inter;
     int rc = 0;
     float *gu = reinterpret_cast<float *>(base);
-    rc = dispatch_linear(p->gu, x, x_dtype, m, nullptr, gu, NNQ_F32, stream, 0, status_dev, fused ? 1 : 0, lin,
+    rc = dispatch_linear(p->gu, x, x_dtype, m, nullptr, gu, NNQ_F32, stream, 0, status_dev, fused || hout ? 1 : 0, lin,
                          hout ? 1 : 0);
     if (rc) return rc;
-    if (hout) return dispatch_linear(p->down, gu, NNQ_F32, m, nullptr, y, y_dtype, stream, 0, status_dev, 2);
+    if (hout && m <= 2) return dispatch_linear(p->down, gu, NNQ_F32, m, nullptr, y, y_dtype, stream, 0, status_dev, 2);
     if (fused) return dispatch_linear(p->down, gu, NNQ_F32, m, nullptr, y, y_dtype, stream, 1, status_dev, 2);
-    float *h = reinterpret_cast<float *>(base + gu_bytes);
-    int e = launch_swiglu(gu, m, I, h, status_dev, stream, p->interleaved8 ? 1 : 0);
+    // (the gate | up GEMM that wrote h has cleared the status, otherwise swiglu_kernel does)
+    float *h = hout ? gu : reinterpret_cast<float *>(base + gu_bytes);
+    int e = hout ? 0 : launch_swiglu(gu, m, I, h, status_dev, stream, p->interleaved8 ? 1 : 0);
     if (e) return hip_fail((hipError_t)e, "swiglu launch");
     rc = dispatch_linear(p->down, h, NNQ_F32, m, nullptr, y, y_dtype, stream, 0, nullptr, 0, lin);
     if (rc) return rc;
@@ -942,12 +953,14 @@ int nnq_mlp_forward(const nnq_mlp *p, const void *x, nnq_dtype x_dtype, int64_t 
     const int64_t I = p->inter;
     // m <= 2: interleaved Q4_K gate | up -> the GEMV writes h = silu(gate) * up and the
     // down GEMV reads h; otherwise the down GEMV takes gate | up and applies SwiGLU while
-    // staging.  m > 2: linear, swiglu_kernel, linear.
-    const bool fused = m <= 2, hout = fused && p->interleaved8;
+    // staging.
+    // m > 2: linear, swiglu_kernel, linear, except that the wide prefill GEMM of an interleaved
+    // gate | up writes h itself.
+    const bool fused = m <= 2, hout = p->interleaved8 && (fused || prefill_swiglu(p->gu, m, x_dtype));
     // one workspace: gate | up [m, 2I] f32 (h [m, I] when hout), h [m, I] f32, the GEMM
     // scratch of either linear, then a misaligned x or y staged
     size_t gu_bytes = 0, h_bytes = 0, xbytes = 0, ybytes = 0;
-    if (!array_bytes(m, (hout ? 1 : 2) * I, 4, &gu_bytes) || !array_bytes(m, fused ? 0 : I, 4, &h_bytes) ||
+    if (!array_bytes(m, (hout ? 1 : 2) * I, 4, &gu_bytes) || !array_bytes(m, fused || hout ? 0 : I, 4, &h_bytes) ||
         !array_bytes(m, k, x_dtype == NNQ_BF16 ? 2 : 4, &xbytes) ||
         !array_bytes(m, p->hidden, y_dtype == NNQ_BF16 ? 2 : 4, &ybytes))
         return size_fail();

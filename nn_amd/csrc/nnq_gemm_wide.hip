@@ -1,4 +1,4 @@
-// Prefill GEMM for Q4_K weights and bf16 activations on gfx950, wide-wave-tile kernel:
+// Prefill GEMM for Q4_K weights on gfx950, wide-wave-tile kernel:
 // Y[m, n] = X[m, k] . W[n, k]^T (+ bias), the arithmetic of QLinear::forward with a batch of
 // tokens (crates/nn-core/src/layers/quantized/linear.rs:366-400; the bf16 result dtype of
 // crates/nn-core/src/dyn_tensor/ops/matmul.rs:37-38).
@@ -16,15 +16,19 @@
 //    16 bytes), while the MFMAs of the previous super-block run; a thread decodes one or two
 //    16-byte pieces of the tile16 code plane (with the row's whole 16-byte header): masked
 //    nibble pairs are f16 subnormals q * 2^-24 (low nibbles) or 16 q * 2^-24 (high nibbles),
-//    times sc or sc / 16, all exact;
+//    times sc or sc / 16, all exact.  With f32 x the pairs come under 0x6400 as 1024 + q or
+//    1024 + 16 q and one packed FMA with sc and -1024 sc (or sc / 16 and -64 sc) makes them
+//    sc * q: the matrix core aligns products by their operands' exponent fields, and next to
+//    the lo parts of x a subnormal B operand would cost the sums low bits;
 //  * each wave's A fragments come from the fragment-major staged activation (one contiguous
 //    1 KB per 16 rows x 32 k, each row's 64 bytes together), PD steps ahead in a register ring;
 //  * the super-block's MFMAs accumulate from zero into `part`; after its last step's MFMAs
-//    for a column tile every lane adds (d * 2^16 * s_n) * part into its totals `tot`, and
+//    for a column tile every lane adds (d * f * s_n) * part into its totals `tot`, and
 //    the min term is one more MFMA per 16 x 16 tile, issued in the first step of the next
 //    super-block: the staged negated sub-block sums of x (f16 hi / lo) against the weight's
 //    aux plane (dmin * m_j * s_n as exact f16 hi / lo), accumulated straight into `tot`
-//    (both carry the column factor 2^16 * s_n);
+//    (both carry the column factor 2^-8 * s_n of sc * q: f = 2^16 for subnormal operands,
+//    2^-8 for normal ones);
 //  * one barrier per super-block (lgkmcnt only: the A prefetches stay in flight).
 // Epilogue: y = tot * 2^8 / s_n * 2^-s_row (+ bias), assembled in LDS and written as 16-byte
 // row chunks; with the K range split, f32 slabs summed in order by gemm_finalize_kernel.
@@ -39,7 +43,6 @@ constexpr int WV = 8;             // waves per workgroup (stacked along M)
 constexpr int MT = 2;             // 16-row MFMA tiles per wave
 constexpr int BM = WV * MT * 16;  // 256 rows per workgroup
 constexpr int NTH = WV * 64;
-constexpr int PD = 3;             // A-fragment prefetch distance in 32-k steps
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
@@ -73,6 +76,9 @@ struct WideArgs {
     void *y;
     float *ysplit;       // [ks][m][n] f32 slabs when ks > 1
     int y_bf16;
+    int swiglu;          // every 16 columns are 8 gates and their 8 ups: y [m][n / 2] f32 gets
+                         //   silu(gate) * up (ks 1, no bias), and *status (if any) NNQ_OK
+    int32_t *status;
     int m, nblk, ntile, ks, nrg;
     int64_t n;
 };
@@ -84,6 +90,13 @@ __device__ __forceinline__ uint32_t pk_mul_bcast(uint32_t a, uint32_t s) {
     const half2v b = HI ? half2v{sv[1], sv[1]} : half2v{sv[0], sv[0]};
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, a) * b);
 }
+// f16 pair FMA a * (s.lo, s.lo) + (o.lo, o.lo) (HI = 0), or with the high halves (HI = 1)
+template <int HI>
+__device__ __forceinline__ uint32_t pk_fma_bcast(uint32_t a, half2v s, half2v o) {
+    const half2v b = HI ? half2v{s[1], s[1]} : half2v{s[0], s[0]};
+    const half2v c = HI ? half2v{o[1], o[1]} : half2v{o[0], o[0]};
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2v, a), b, c));
+}
 
 // One 16-byte piece of a tile16 group: bytes 16 h .. 16 h + 15 of row r's 32-byte group p,
 // which consumer lanes G = 2h and 2h + 1 take 8 bytes each of: their low nibbles are
@@ -91,6 +104,7 @@ __device__ __forceinline__ uint32_t pk_mul_bcast(uint32_t a, uint32_t s) {
 // sub-block 2p + 1 (step 2p + 1).  out[g][hh] is the B fragment slice of lane G = 2h + g at
 // step 2p + hh.  h is the row's header (BlockQ4K: d | dmin, scales[12]; get_scale_min_k4,
 // crates/nn-core/src/layers/quantized/linear.rs:166-176).
+template <int P>
 __device__ __forceinline__ void decode_piece(u32x4 raw, u32x4 h, int p, u32x4 out[2][2]) {
     const uint32_t sc03 = h[1] & 0x3F3F3F3Fu;
     const uint32_t sc47 = (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u);
@@ -100,14 +114,29 @@ __device__ __forceinline__ void decode_piece(u32x4 raw, u32x4 h, int p, u32x4 ou
     const uint32_t biased = 0x64006400u | (pair & 0xFFu) | ((pair & 0xFF00u) << 8);
     const half2v sh = (__builtin_bit_cast(half2v, biased) - half2v{(_Float16)1024.0f, (_Float16)1024.0f}) *
                       half2v{(_Float16)1.0f, (_Float16)0.0625f};
-    const uint32_t sw = __builtin_bit_cast(uint32_t, sh);
+    if constexpr (P == 1) {
+        const uint32_t sw = __builtin_bit_cast(uint32_t, sh);
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const uint32_t w0 = raw[2 * g], w1 = raw[2 * g + 1], w0s = w0 >> 8, w1s = w1 >> 8;
+            out[g][0] = u32x4{pk_mul_bcast<0>(w0 & 0x000F000Fu, sw), pk_mul_bcast<0>(w0s & 0x000F000Fu, sw),
+                              pk_mul_bcast<0>(w1 & 0x000F000Fu, sw), pk_mul_bcast<0>(w1s & 0x000F000Fu, sw)};
+            out[g][1] = u32x4{pk_mul_bcast<1>(w0 & 0x00F000F0u, sw), pk_mul_bcast<1>(w0s & 0x00F000F0u, sw),
+                              pk_mul_bcast<1>(w1 & 0x00F000F0u, sw), pk_mul_bcast<1>(w1s & 0x00F000F0u, sw)};
+        }
+        return;
+    }
+    // codes under 0x6400 are 1024 + q (low nibbles) and 1024 + 16 q (high): the 1024 leaves as
+    // -1024 sc and -64 sc in the same FMA (at most 64512, exact)
+    const half2v so = sh * half2v{(_Float16)-1024.0f, (_Float16)-1024.0f};
+    constexpr uint32_t LO = 0x000F000Fu, HI = 0x00F000F0u, B = 0x64006400u;
 #pragma unroll
     for (int g = 0; g < 2; g++) {
         const uint32_t w0 = raw[2 * g], w1 = raw[2 * g + 1], w0s = w0 >> 8, w1s = w1 >> 8;
-        out[g][0] = u32x4{pk_mul_bcast<0>(w0 & 0x000F000Fu, sw), pk_mul_bcast<0>(w0s & 0x000F000Fu, sw),
-                          pk_mul_bcast<0>(w1 & 0x000F000Fu, sw), pk_mul_bcast<0>(w1s & 0x000F000Fu, sw)};
-        out[g][1] = u32x4{pk_mul_bcast<1>(w0 & 0x00F000F0u, sw), pk_mul_bcast<1>(w0s & 0x00F000F0u, sw),
-                          pk_mul_bcast<1>(w1 & 0x00F000F0u, sw), pk_mul_bcast<1>(w1s & 0x00F000F0u, sw)};
+        out[g][0] = u32x4{pk_fma_bcast<0>((w0 & LO) | B, sh, so), pk_fma_bcast<0>((w0s & LO) | B, sh, so),
+                          pk_fma_bcast<0>((w1 & LO) | B, sh, so), pk_fma_bcast<0>((w1s & LO) | B, sh, so)};
+        out[g][1] = u32x4{pk_fma_bcast<1>((w0 & HI) | B, sh, so), pk_fma_bcast<1>((w0s & HI) | B, sh, so),
+                          pk_fma_bcast<1>((w1 & HI) | B, sh, so), pk_fma_bcast<1>((w1s & HI) | B, sh, so)};
     }
 }
 
@@ -125,10 +154,13 @@ __device__ __forceinline__ uint32_t bload1(__amdgpu_buffer_rsrc_t r, int voff, i
     return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
 }
 
-template <int NT>
+// P: activation planes (1: f16 of bf16 x, exact; 2: the f16 hi and lo parts of f32 x, two MFMAs
+// per step and tile over the same B fragment)
+template <int NT, int P>
 __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     using C = Wide<NT>;
-    constexpr int PPT = C::PPT;
+    constexpr int PPT = C::PPT, PD = P == 1 ? 3 : 2;  // A-fragment prefetch distance in 32-k steps
+    constexpr int RING = P == 1 ? PD + 1 : PD + 2;    // (a divisor of the 8 steps)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -148,11 +180,13 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     // Buffer resources over wave-uniform bases; per-lane 32-bit offsets, per-step scalar
     // offsets.  A fragments: the wave's two row groups (past the last: clamped, not stored),
     // steps [sb0 * 8, sb0 * 8 + nsteps); reads past the range (prefetch beyond the end) give 0.
-    __amdgpu_buffer_rsrc_t ra[MT], rxs[MT];
+    __amdgpu_buffer_rsrc_t ra[MT][P], rxs[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const int rg = min(rt * (BM / 16) + wv * MT + mt, a.nrg - 1);
-        ra[mt] = rsrc(a.xa + ((size_t)rg * nblk * 8 + (size_t)sb0 * 8) * 64, (int64_t)nsteps * 1024);
+#pragma unroll
+        for (int pl = 0; pl < P; pl++)
+            ra[mt][pl] = rsrc(a.xa + (((size_t)pl * a.nrg + rg) * nblk * 8 + (size_t)sb0 * 8) * 64, (int64_t)nsteps * 1024);
         rxs[mt] = rsrc(a.xs + ((size_t)rg * nblk + sb0) * 64, (int64_t)nsb * 1024);
     }
     const int loff = (c16 * 4 + G) * 16;  // lane (G, r) of a fragment: row r's 16 bytes G
@@ -165,14 +199,14 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     const int qoff = ph * 1024 + (16 * pgp + c16) * 16, hoff = c16 * 16;
     const int xoff = (lane >> 5) * 256 + c16 * 16;
     const int tw = __builtin_amdgcn_readfirstlane(tid >> 7);  // tile of this thread's first piece
-    // per column: 2^16 * s_n, the totals' unit (s_n a normal power of two), and the epilogue's
+    // per column: 2^16 or 2^-8 times s_n, what brings the partial sums to the totals' unit (s_n a normal power of two), and the epilogue's
     // factors, loaded now: 2^8 / s_n and the bias per column, 2^-s_row per row
     const float *srow = reinterpret_cast<const float *>(a.aux + (size_t)a.ntile * nblk * 512);
     float f1[NT], f2[NT], bc[NT], rb[MT][4];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
         const uint32_t eb = __float_as_uint(srow[(size_t)(t0 + nt) * 16 + c16]) >> 23;
-        f1[nt] = __uint_as_float((eb + 16u) << 23);
+        f1[nt] = __uint_as_float((P == 1 ? eb + 16u : eb - 8u) << 23);
         f2[nt] = __uint_as_float((262u - eb) << 23);
         bc[nt] = (a.bias && a.ks == 1) ? a.bias[(int64_t)(t0 + nt) * 16 + c16] : 0.0f;
     }
@@ -207,7 +241,7 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
         // here: reused as a temporary while the load is in flight, it would make the wave
         // wait for that (HBM-latency) load at once
         asm volatile("" ::"v"(hd[j][2]));
-        decode_piece(raw[j], hd[j], pgp, o);
+        decode_piece<P>(raw[j], hd[j], pgp, o);
 #pragma unroll
         for (int g = 0; g < 2; g++)
 #pragma unroll
@@ -224,11 +258,13 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
 
     // prologue: super-block 0 into buffer 0, the A ring filled
     load_raw(0);
-    u32x4 af[PD + 1][MT];
+    u32x4 af[RING][MT][P];
 #pragma unroll
     for (int s = 0; s < PD; s++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) af[s][mt] = bload4(ra[mt], loff, s * 1024);
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int pl = 0; pl < P; pl++) af[s][mt][pl] = bload4(ra[mt][pl], loff, s * 1024);
 #pragma unroll
     for (int j = 0; j < PPT; j++) store_piece(smem, j);
     if (wv < NT) *reinterpret_cast<u32x4 *>(smem + C::AUX_OFF + (wv * 64 + lane) * 16) = auxv;
@@ -261,14 +297,17 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
         for (int s = 0; s < 8; s++) {
             // A fragments PD steps ahead (past the range: zeros, never used)
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) af[(s + PD) % (PD + 1)][mt] = bload4(ra[mt], loff, (sb * 8 + s + PD) * 1024);
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int pl = 0; pl < P; pl++)
+                    af[(s + PD) % RING][mt][pl] = bload4(ra[mt][pl], loff, (sb * 8 + s + PD) * 1024);
             __builtin_amdgcn_sched_barrier(0);
             u32x4 bf[NT];
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) bf[nt] = *reinterpret_cast<const u32x4 *>(cur + ((nt * 8 + s) * 64 + lane) * 16);
             if (s == 0 && sb > 0) min_term(sb - 1, xsp_prev);
             if (s == 6) {
-                // the super-block's factor d per column (2^16 * s_n folded in)
+                // the super-block's factor d per column (f1 folded in)
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++)
                     dn[nt] = *reinterpret_cast<const float *>(cur + C::D_OFF + (nt * 16 + c16) * 4) * f1[nt];
@@ -276,9 +315,12 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    part[mt][nt] = mfma16x16x32_f16(af[s % (PD + 1)][mt], bf[nt],
-                                                    s == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : part[mt][nt]);
+                for (int pl = P - 1; pl >= 0; pl--)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+                        part[mt][nt] = mfma16x16x32_f16(af[s % RING][mt][pl], bf[nt],
+                                                        s == 0 && pl == P - 1 ? floatx4{0.f, 0.f, 0.f, 0.f}
+                                                                              : part[mt][nt]);
                 if (s == 7) {
 #pragma unroll
                     for (int mt = 0; mt < MT; mt++)
@@ -306,7 +348,7 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     __builtin_amdgcn_s_barrier();
 
     // epilogue: y = tot * 2^8 / s_n * 2^-s_row (+ bias), assembled in LDS, 16-byte row chunks
-    const bool f32out = a.ks > 1 || !a.y_bf16;
+    const bool f32out = a.ks > 1 || a.swiglu || !a.y_bf16;
     const int es = f32out ? 4 : 2, rs = C::BN * es + 16;
     if (f32out) {
 #pragma unroll
@@ -329,8 +371,23 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
-    const int cpr = C::BN * es / 16;  // 16-byte chunks per row
     const int m0 = rt * BM;
+    if (a.swiglu) {
+        if (a.status && bid == 0 && tid == 0) *a.status = NNQ_OK;
+        // h = silu(g) * u (crates/nn-qwen3/src/layers.rs:19-48, math.rs:140), four columns a thread
+        for (int c = tid; c < BM * NT * 2; c += NTH) {
+            const int rl = c / (NT * 2), q = c - rl * (NT * 2);
+            if (m0 + rl >= a.m) break;  // rows run in order
+            const unsigned char *p = smem + rl * rs + (q >> 1) * 64 + (q & 1) * 16;
+            const floatx4 g = *reinterpret_cast<const floatx4 *>(p), u = *reinterpret_cast<const floatx4 *>(p + 32);
+            floatx4 h;
+#pragma unroll
+            for (int e = 0; e < 4; e++) h[e] = g[e] / (1.0f + expf(-g[e])) * u[e];
+            *reinterpret_cast<floatx4 *>(reinterpret_cast<float *>(a.y) + (int64_t)(m0 + rl) * (a.n / 2) + t0 * 8 + q * 4) = h;
+        }
+        return;
+    }
+    const int cpr = C::BN * es / 16;  // 16-byte chunks per row
     unsigned char *ybase = a.ks > 1 ? reinterpret_cast<unsigned char *>(a.ysplit + (int64_t)kp * a.m * a.n)
                                     : reinterpret_cast<unsigned char *>(a.y);
     for (int c = tid; c < BM * cpr; c += NTH) {
@@ -512,10 +569,11 @@ __global__ __launch_bounds__(W * 64) void gemm_q4k_skinny_kernel(WideArgs a) {
 // 64-byte segment).  The min-term operands: per (row group, super-block) one fragment in
 // the same order whose lane 16 G + r holds the f16 hi (G even) or lo (G odd) parts of
 // -2^-8 * sum(x * 2^s_row) over the row's eight 32-element sub-blocks.  Rows past M
-// (padding to 16) are written as zeros.
+// (padding to 16) are written as zeros.  f32 x (XF): the f16 hi part as above, and the lo
+// part x * 2^s_row - hi in a second plane after the first.
 // ---------------------------------------------------------------------------------
-template <int NG, bool XS>
-__global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const uint16_t *x, int64_t m, int64_t k, u32x4 *xa,
+template <int NG, bool XS, bool XF>
+__global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const void *xv, int64_t m, int64_t k, u32x4 *xa,
                                                               u32x4 *xs, float *rowback) {
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wvi = tid >> 6;
@@ -524,18 +582,35 @@ __global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const uint16_t *x,
     const bool valid = row < m;
     const int64_t ng = k / 8, nks = k / 32;
     const int g = (int)(row >> 4), r = (int)(row & 15);
-    u32x4 w[NG];
+    const u32x4 none = {0u, 0u, 0u, 0u};
+    float v[NG][8];
 #pragma unroll
     for (int j = 0; j < NG; j++) {
         const int64_t c = tid + 512 * j;
-        w[j] = (valid && c < ng) ? *reinterpret_cast<const u32x4 *>(x + row * k + 8 * c) : u32x4{0u, 0u, 0u, 0u};
+        const bool in = valid && c < ng;
+        if constexpr (XF) {
+            const float *x = reinterpret_cast<const float *>(xv) + row * k + 8 * c;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const u32x4 w = in ? *reinterpret_cast<const u32x4 *>(x + 4 * h) : none;
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[j][4 * h + i] = __uint_as_float(w[i]);
+            }
+        } else {
+            const uint16_t *x = reinterpret_cast<const uint16_t *>(xv) + row * k + 8 * c;
+            const u32x4 w = in ? *reinterpret_cast<const u32x4 *>(x) : none;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v[j][2 * i] = bf16_to_f32(w[i] & 0xFFFFu);
+                v[j][2 * i + 1] = bf16_to_f32(w[i] >> 16);
+            }
+        }
     }
     float amax = 0.0f;
 #pragma unroll
     for (int j = 0; j < NG; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            amax = fmaxf(amax, fmaxf(fabsf(bf16_to_f32(w[j][i] & 0xFFFFu)), fabsf(bf16_to_f32(w[j][i] >> 16))));
+        for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[j][i]));
     amax = wave_max(amax);
     if (lane == 0) wred[wvi] = amax;
     __syncthreads();
@@ -548,19 +623,25 @@ __global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const uint16_t *x,
     for (int j = 0; j < NG; j++) {
         const int64_t c = tid + 512 * j;  // chunk of 8: step c / 4, lane group c % 4
         if (j * 512 < ng) {               // wave-uniform: whole groups of 64 chunks (k % 512 == 0)
-            uint32_t h[4];
+            uint32_t h[4], l[4];
             float sum = 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const float a0 = bf16_to_f32(w[j][i] & 0xFFFFu) * s, a1 = bf16_to_f32(w[j][i] >> 16) * s;
+                const float a0 = v[j][2 * i] * s, a1 = v[j][2 * i + 1] * s;
                 sum += a0 + a1;
-                h[i] = f32_to_f16_bits(a0) | (f32_to_f16_bits(a1) << 16);
+                uint32_t h0, h1, l0, l1;
+                split_f16(a0, h0, l0);
+                split_f16(a1, h1, l1);
+                h[i] = h0 | (h1 << 16);
+                l[i] = l0 | (l1 << 16);
             }
             // the sub-block's sum over its four chunks (lanes c .. c + 3 of one quad)
             sum += dpp_xor1(sum);
             sum += dpp_xor2(sum);
             if (c < ng) {
-                xa[((int64_t)g * nks + c / 4) * 64 + r * 4 + (c % 4)] = u32x4{h[0], h[1], h[2], h[3]};
+                const int64_t o = ((int64_t)g * nks + c / 4) * 64 + r * 4 + (c % 4);
+                xa[o] = u32x4{h[0], h[1], h[2], h[3]};
+                if constexpr (XF) xa[(int64_t)gridDim.x / 16 * nks * 64 + o] = u32x4{l[0], l[1], l[2], l[3]};
                 if ((c & 3) == 0) sums[c / 4] = sum;
             }
         }
@@ -590,32 +671,45 @@ __global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const uint16_t *x,
 
 }  // namespace
 
-// The wide kernel's shape rules: bf16 activations, more than 128 rows (smaller batches are
-// HBM-bound and take the other kernels), whole 16-row weight tiles and a 16-byte aligned
-// output (the epilogue writes 16-byte row chunks), K <= 4096 * 3 (the staging
-// keeps the row in one workgroup's registers and its sub-block sums in LDS), and enough workgroups to fill
-// the CUs: 96-column tiles when they give at least 192 workgroups, else 64-column tiles
-// (an even super-block count) when they give 128 with the K range split in two below 256.
-// Returns the column tiles per workgroup (6 or 4; 0: the ring kernel takes the shape) and
-// the K split.
+// The wide kernel's shape rules: more than 128 rows (below, half of a 256-row tile or more is
+// padding: f32 x, 100 x 4096 x 12288 109 us against the ring's 51), whole 16-row weight tiles
+// and a 16-byte aligned output (the epilogue writes 16-byte row chunks), K <= 4096 * 3 (the
+// staging keeps the row in one workgroup's registers and its sub-block sums in LDS), and at
+// least 128 workgroups.  Column tiles per workgroup (6 or 4) and K split (1 to 4 equal parts
+// of whole super-blocks) are the ones with the least estimated time: rounds of workgroups over
+// the CUs, times super-blocks, times the measured time of one (us, 6 and 4 tiles: bf16 x 3.8
+// and 3.0, f32 x 6.1 and 5.2), plus the slabs' write, read and launch.  512 rows of f32 x take
+// 106 us at 12288 x 4096 (6 tiles; the ring kernel over two planes 153) and 134 at 4096 x 12288
+// (4 tiles, K in two; 155); 203 rows at 12288 x 4096 take 6 tiles and K in two (256 workgroups).
+// Returns the column tiles per workgroup (0: the ring kernel takes the shape) and the K split.
 int gemm_wide_plan(const GemmArgs &a, int *ks) {
-    if (a.blk || !a.x_bf16 || a.m <= 128 || a.k > 4096 * 3 || a.n != a.ntile * 16 ||
-        (reinterpret_cast<uintptr_t>(a.y) & 15))
-        return 0;
+    if (a.blk || a.m <= 128 || a.k > 4096 * 3 || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
     const int64_t nrt = (a.m + BM - 1) / BM;
-    if (a.ntile % 6 == 0 && nrt * (a.ntile / 6) >= 192) {
-        if (ks) *ks = 1;
-        return 6;
-    }
-    if (a.ntile % 4 == 0) {
-        const int64_t wg = nrt * (a.ntile / 4);
-        const int split = wg >= 256 ? 1 : 2;
-        if (wg * split >= 128 && a.nblk % split == 0 && a.nblk / split >= 2) {
-            if (ks) *ks = split;
-            return 4;
+    const float sb_us[2][2] = {{3.8f, 3.0f}, {6.1f, 5.2f}};
+    float best = 0.0f;
+    int nt = 0;
+    for (int i = 0; i < 2; i++) {
+        const int c = i == 0 ? 6 : 4;
+        if (a.ntile % c) continue;
+        for (int split = 1; split <= 4; split++) {
+            const int64_t wg = nrt * (a.ntile / c) * split;
+            if (wg < 128 || a.nblk % split || a.nblk / split < 2) continue;
+            const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(a.m * a.n) * 4.0f / 4.0e6f : 0.0f;
+            const float us = (float)((wg + 255) / 256 * (a.nblk / split)) * sb_us[a.x_bf16 ? 0 : 1][i] + slabs;
+            if (!nt || us < best) {
+                best = us;
+                nt = c;
+                if (ks) *ks = split;
+            }
         }
     }
-    return 0;
+    return nt;
+}
+
+// whether the call can write silu(gate) * up (swiglu_out) from the wide kernel's epilogue
+bool gemm_wide_swiglu(const GemmArgs &a) {
+    int ks = 0;
+    return gemm_wide_plan(a, &ks) && ks == 1;
 }
 
 // The skinny kernel's shape rules: bf16 activations, 17 to 32 rows (fewer: the thin
@@ -639,7 +733,7 @@ size_t gemm_wide_scratch(const GemmArgs &a, GemmScratch *s, uint8_t *base) {
     if (!gemm_skinny_plan(a, nullptr, nullptr)) gemm_wide_plan(a, &ks);
     size_t off = 0;
     if (s) s->xh = reinterpret_cast<uint16_t *>(base + off);
-    off += al((size_t)nrg * 16 * a.k * 2);
+    off += al((size_t)(a.x_bf16 ? 1 : 2) * nrg * 16 * a.k * 2);
     if (s) s->xs = reinterpret_cast<uint16_t *>(base + off);
     off += al((size_t)nrg * (a.k / 256) * 1024);
     if (s) s->rowback = reinterpret_cast<float *>(base + off);
@@ -655,18 +749,18 @@ size_t gemm_wide_scratch(const GemmArgs &a, GemmScratch *s, uint8_t *base) {
     return off;
 }
 
-template <int NT>
+template <int NT, int P>
 static int launch_wide_nt(const WideArgs &w, hipStream_t st) {
     using C = Wide<NT>;
     static bool attr_set = false;  // idempotent attribute write; races only repeat it
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q4k_wide_kernel<NT>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q4k_wide_kernel<NT, P>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS);
         if (e != hipSuccess) return (int)e;
         attr_set = true;
     }
     const int total = (w.ntile / NT) * ((w.m + BM - 1) / BM) * w.ks;
-    hipLaunchKernelGGL((gemm_q4k_wide_kernel<NT>), dim3((unsigned)total), dim3(NTH), C::LDS, st, w);
+    hipLaunchKernelGGL((gemm_q4k_wide_kernel<NT, P>), dim3((unsigned)total), dim3(NTH), C::LDS, st, w);
     return (int)hipGetLastError();
 }
 
@@ -684,22 +778,26 @@ static int launch_skinny_cfg(const WideArgs &w, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-int launch_stage_wide(const uint16_t *x, int64_t m, int64_t k, void *xa, void *xs, float *rowback, void *stream) {
+template <int NG>
+static void launch_stage_ng(const void *x, int x_bf16, dim3 sg, int64_t m, int64_t k, u32x4 *fa, u32x4 *fs, float *rowback,
+                            hipStream_t st) {
+    if (!x_bf16)
+        hipLaunchKernelGGL((gemm_stage_wide_kernel<NG, true, true>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
+    else if (fs)
+        hipLaunchKernelGGL((gemm_stage_wide_kernel<NG, true, false>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
+    else
+        hipLaunchKernelGGL((gemm_stage_wide_kernel<NG, false, false>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
+}
+
+int launch_stage_wide(const void *x, int x_bf16, int64_t m, int64_t k, void *xa, void *xs, float *rowback, void *stream) {
     const dim3 sg((unsigned)((m + 15) / 16 * 16));
     hipStream_t st = (hipStream_t)stream;
     auto fa = reinterpret_cast<u32x4 *>(xa), fs = reinterpret_cast<u32x4 *>(xs);
-    if (k > 4096 * 3 || k % 256) return (int)hipErrorInvalidValue;
-    if (k <= 4096) {
-        if (xs)
-            hipLaunchKernelGGL((gemm_stage_wide_kernel<1, true>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
-        else
-            hipLaunchKernelGGL((gemm_stage_wide_kernel<1, false>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
-    } else {
-        if (xs)
-            hipLaunchKernelGGL((gemm_stage_wide_kernel<3, true>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
-        else
-            hipLaunchKernelGGL((gemm_stage_wide_kernel<3, false>), sg, dim3(512), 0, st, x, m, k, fa, fs, rowback);
-    }
+    if (k > 4096 * 3 || k % 256 || (!x_bf16 && !xs)) return (int)hipErrorInvalidValue;
+    if (k <= 4096)
+        launch_stage_ng<1>(x, x_bf16, sg, m, k, fa, fs, rowback, st);
+    else
+        launch_stage_ng<3>(x, x_bf16, sg, m, k, fa, fs, rowback, st);
     return (int)hipGetLastError();
 }
 
@@ -712,8 +810,7 @@ int launch_gemm_wide(const GemmArgs &a, const GemmScratch &sc, void *stream) {
     const int64_t nrg = (a.m + 15) / 16;
     auto xa = reinterpret_cast<u32x4 *>(sc.xh);
     auto xs = reinterpret_cast<u32x4 *>(sc.xs);
-    auto xin = reinterpret_cast<const uint16_t *>(a.x);
-    int e = launch_stage_wide(xin, a.m, a.k, xa, xs, sc.rowback, stream);
+    int e = launch_stage_wide(a.x, a.x_bf16, a.m, a.k, xa, xs, sc.rowback, stream);
     if (e) return e;
     WideArgs w{};
     w.qs = a.qs;
@@ -726,6 +823,9 @@ int launch_gemm_wide(const GemmArgs &a, const GemmScratch &sc, void *stream) {
     w.y = a.y;
     w.ysplit = sc.ysplit;
     w.y_bf16 = a.y_bf16;
+    w.swiglu = a.swiglu_out;
+    w.status = a.status;
+    if (a.swiglu_out && (skinny || ks != 1 || a.bias)) return (int)hipErrorInvalidValue;
     w.m = (int)a.m;
     w.n = a.n;
     w.nblk = (int)a.nblk;
@@ -735,7 +835,10 @@ int launch_gemm_wide(const GemmArgs &a, const GemmScratch &sc, void *stream) {
     if (skinny) {
         return launch_skinny_cfg<3, 2, 8>(w, st);  // the plan: 17 to 32 rows, three tiles, eight waves
     }
-    e = nt == 6 ? launch_wide_nt<6>(w, st) : launch_wide_nt<4>(w, st);
+    if (a.x_bf16)
+        e = nt == 6 ? launch_wide_nt<6, 1>(w, st) : launch_wide_nt<4, 1>(w, st);
+    else
+        e = nt == 6 ? launch_wide_nt<6, 2>(w, st) : launch_wide_nt<4, 2>(w, st);
     if (e || ks == 1) return e;
     return launch_gemm_finalize(sc.ysplit, ks, a.bias, a.y, a.y_bf16, a.m, a.n, stream);
 }

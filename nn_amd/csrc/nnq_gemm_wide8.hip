@@ -331,7 +331,7 @@ int launch_gemm_wide8(const GemmArgs &a, const GemmScratch &sc, void *stream) {
     if (!nt || sc.ksplit != ks || (ks > 1 && !sc.ysplit)) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
     const int64_t nrg = (a.m + 15) / 16;
-    int e = launch_stage_wide(reinterpret_cast<const uint16_t *>(a.x), a.m, a.k, sc.xh, nullptr, sc.rowback, stream);
+    int e = launch_stage_wide(a.x, 1, a.m, a.k, sc.xh, nullptr, sc.rowback, stream);
     if (e) return e;
     Wide8Args w{};
     w.qs = a.qs;

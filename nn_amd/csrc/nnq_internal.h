@@ -141,6 +141,9 @@ struct GemmArgs {
     int64_t n, k, m;
     int64_t ntile, nblk;
     void *scratch;
+    int swiglu_out;  // wide Q4_K kernel without a K split only (gemm_wide_swiglu): y [m, n / 2] f32
+                     //   gets silu(gate) * up of columns that come as 8 gates, then their 8 ups;
+    int32_t *status; //   status (optional) is set to NNQ_OK
     int blk;  // 0: Q4_K; NNQ_FMT_Q8_0 / NNQ_FMT_Q6_K: the block-scaled GEMM (nnq_gemm_blk.hip)
 };
 int launch_gemm_q4k(const GemmArgs &a, void *stream);
@@ -171,19 +174,21 @@ struct GemmScratch {
 // the kernel; bn and bm, when given, receive the tile width and height), and its launch
 int gemm_ring_plan(const GemmArgs &a, int *bn, int *bm = nullptr);
 int launch_gemm_ring(const GemmArgs &a, const GemmScratch &sc, void *stream);
-// wide-wave-tile kernel (nnq_gemm_wide.hip; bf16 activations, more than 128 rows): its
+// wide-wave-tile kernel (nnq_gemm_wide.hip; more than 128 rows): its
 // column tiles per workgroup (0: the shape does not fit) and K split, its scratch (the
 // fragment-major staged activation in xh, min-term operands in xs, rowback, split slabs;
 // s null: sizes only) and its launch (staging, kernel, and with a K split the slab sum)
 int gemm_wide_plan(const GemmArgs &a, int *ks);
+bool gemm_wide_swiglu(const GemmArgs &a);
 // the skinny kernel (same file and staging; bf16 activations, 17 to 32 rows): whether it
 // takes the shape, with its tiles per workgroup R and waves W
 int gemm_skinny_plan(const GemmArgs &a, int *R, int *W);
 size_t gemm_wide_scratch(const GemmArgs &a, GemmScratch *s, uint8_t *base);
 int launch_gemm_wide(const GemmArgs &a, const GemmScratch &sc, void *stream);
-// the wide kernels' activation staging (bf16 x, K a multiple of 256 up to 12288): f16 of
-// x * 2^s_row in fragment order, 2^-s_row per row, and (xs given) the Q4_K min-term operands
-int launch_stage_wide(const uint16_t *x, int64_t m, int64_t k, void *xa, void *xs, float *rowback, void *stream);
+// the wide kernels' activation staging (K a multiple of 256 up to 12288): f16 of x * 2^s_row
+// in fragment order (f32 x: a hi and a lo plane), 2^-s_row per row, and (xs given, always with
+// f32 x) the Q4_K min-term operands
+int launch_stage_wide(const void *x, int x_bf16, int64_t m, int64_t k, void *xa, void *xs, float *rowback, void *stream);
 // Q8_0 wide kernel (nnq_gemm_wide8.hip): column tiles per workgroup (0: not its shape) and
 // K split; its scratch; the staging and the kernel (and the slab sum with a split)
 int gemm_wide8_plan(const GemmArgs &a, int *ks);

@@ -66,3 +66,49 @@ def test_wide_row_scales(O, dev):
     err = np.abs(g - r).max(axis=1) / np.abs(r).max(axis=1)
     print(f"row-scale sweep: worst per-row normwise {err.max():.2e}")
     assert err.max() <= 1e-3
+
+
+# f32 activations (hi + lo planes) on the wide kernel: one row past its lower limit, ragged row
+# tiles, both column-tile widths, K split two to four ways and not at all, K of the staging's
+# limit.  Bar: max |error| <= 2e-5 of the output's rms: f32 sums over K <= 12288 of products
+# that keep 22 bits of x (2.3e-6 measured at 512 x 4096 x 12288).
+@pytest.mark.parametrize("m,n,k", [(129, 3072, 1024), (203, 12288, 512), (300, 6144, 2048), (513, 4096, 1280),
+                                   (256, 1024, 12288), (700, 1920, 768)])
+def test_wide_f32_activations(dev, m, n, k):
+    import nn_amd
+    w = make_weight("q4_k", nn_amd.quantize_q4_k(nn_amd.synth_normal(m, 1, (n, k), 0.02)), n, k)
+    x = torch.from_numpy(nn_amd.synth_normal(m, 2, (m, k), 1.0)).to(dev)
+    x[5] *= 1e-20
+    x[7] = 0.0
+    bias = torch.from_numpy(nn_amd.synth_normal(m, 3, (n,), 0.5)).to(dev)
+    y = nn_amd.quantized_linear(x, w, bias)
+    assert torch.equal(y, nn_amd.quantized_linear(x, w, bias)), "repeated calls must agree bit for bit"
+    ref = x.double() @ w.dequantize().double().t() + bias.double()
+    err = ((y.double() - ref).abs().amax(1) / ref.pow(2).mean(1).sqrt()).max().item()
+    assert err <= 2e-5, f"{m}x{n}x{k}: {err:.2e} of the row's rms"
+    yb = nn_amd.quantized_linear(x, w, bias, out_dtype=torch.bfloat16)
+    assert torch.equal(yb, y.to(torch.bfloat16)), "bf16 output: the f32 result rounded once"
+
+
+@pytest.mark.parametrize("m,hidden,inter,xdt", [(129, 512, 6144, torch.bfloat16), (300, 1024, 3072, torch.float32),
+                                               (600, 512, 2048, torch.bfloat16)])
+def test_prefill_mlp_swiglu_epilogue(dev, m, hidden, inter, xdt):
+    """The gate | up GEMM that writes silu(gate) * up itself, against the three linears: h differs by
+    f32 rounding only, so the outputs agree to 1e-5 of their rms; a NaN row is flagged and stays
+    in its row."""
+    import nn_amd
+    q = [nn_amd.quantize_q4_k(nn_amd.synth_normal(5, i, s, 0.02))
+         for i, s in ((1, (inter, hidden)), (2, (inter, hidden)), (3, (hidden, inter)))]
+    mlp = nn_amd.QuantizedMLP(*q, nn_amd.QuantType.Q4_K, hidden, inter)
+    g, u, d = (make_weight("q4_k", b, *s) for b, s in zip(q, ((inter, hidden), (inter, hidden), (hidden, inter))))
+    x = torch.from_numpy(nn_amd.synth_normal(5, 4, (m, hidden), 1.0)).to(dev).to(xdt)
+    y = mlp.forward(x)
+    gate, up = nn_amd.quantized_linear(x, g).double(), nn_amd.quantized_linear(x, u).double()
+    ref = (gate * torch.sigmoid(gate) * up) @ d.dequantize().double().t()
+    assert (y.double() - ref).abs().max().item() <= 1e-5 * ref.pow(2).mean().sqrt().item()
+    x[11, 3] = float("nan")
+    z = mlp.forward(x, check=False)
+    keep = torch.arange(m) != 11
+    assert torch.equal(z[keep], y[keep]) and torch.isnan(z[11]).all()
+    with pytest.raises(nn_amd.NonFiniteData):
+        mlp.forward(x)
