@@ -178,6 +178,10 @@ int nnq_argmax_f32(const float *logits, int64_t n, uint32_t *idx, int32_t *statu
  * crates/nn-core/src/dyn_tensor/ops_ext/argreduce.rs:105-118). */
 int nnq_linear_argmax(const nnq_weight *w, const float *x, int64_t k, const float *bias, int64_t bias_len,
                       float *logits, uint32_t *idx, int32_t *status_dev, void *stream);
+/* The same with the index as a 64-bit integer, the index type of tensor libraries, so that no
+ * conversion launch follows. */
+int nnq_linear_argmax_i64(const nnq_weight *w, const float *x, int64_t k, const float *bias, int64_t bias_len,
+                          float *logits, int64_t *idx, int32_t *status_dev, void *stream);
 
 /* ---- token sampling ------------------------------------------------------------- */
 

@@ -39,6 +39,8 @@ SIGNATURES = {
     "nnq_argmax_f32": (c_int, [c_void_p, c_i64, c_void_p, c_void_p, c_void_p]),
     "nnq_linear_argmax": (c_int, [c_void_p, c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_void_p, c_void_p,
                                   c_void_p]),
+    "nnq_linear_argmax_i64": (c_int, [c_void_p, c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_void_p, c_void_p,
+                                      c_void_p]),
     "nnq_moe_create": (c_int, [c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                ctypes.POINTER(c_void_p)]),
     "nnq_moe_destroy": (c_int, [c_void_p]),

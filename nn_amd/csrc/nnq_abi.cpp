@@ -664,11 +664,14 @@ int nnq_argmax_f32(const float *logits, int64_t n, uint32_t *idx, int32_t *statu
     return NNQ_OK;
 }
 
-int nnq_linear_argmax(const nnq_weight *w, const float *x, int64_t k, const float *bias, int64_t bias_len,
-                      float *logits, uint32_t *idx, int32_t *status_dev, void *stream) {
+}  // extern "C"
+
+// nnq_linear_argmax and nnq_linear_argmax_i64: the index to idx or idx64
+static int linear_argmax(const nnq_weight *w, const float *x, int64_t k, const float *bias, int64_t bias_len,
+                         float *logits, uint32_t *idx, int64_t *idx64, int32_t *status_dev, void *stream) {
     int rc = check_linear(w, x, NNQ_F32, 1, k, bias, bias_len, logits, NNQ_F32);
     if (rc) return rc;
-    if (!idx) return fail(NNQ_ERR_INVALID_ARGUMENT, "idx is null");
+    if (!idx && !idx64) return fail(NNQ_ERR_INVALID_ARGUMENT, "idx is null");
     if (misaligned_out(logits)) return fail(NNQ_ERR_INVALID_ARGUMENT, "logits must be 4-byte aligned");
     const Layout &L = w->L;
     const bool xm = misaligned_in(x);
@@ -700,9 +703,21 @@ int nnq_linear_argmax(const nnq_weight *w, const float *x, int64_t k, const floa
     a.argmax_count = &nkeys;
     int e = launch_gemv(L.fmt, a, stream);
     if (e) return hip_fail((hipError_t)e, "gemv launch");
-    e = launch_argmax_final(a.argmax_partial, nkeys, idx, status_dev, stream);
+    e = launch_argmax_final(a.argmax_partial, nkeys, idx, idx64, status_dev, stream);
     if (e) return hip_fail((hipError_t)e, "argmax launch");
     return NNQ_OK;
+}
+
+extern "C" {
+
+int nnq_linear_argmax(const nnq_weight *w, const float *x, int64_t k, const float *bias, int64_t bias_len,
+                      float *logits, uint32_t *idx, int32_t *status_dev, void *stream) {
+    return linear_argmax(w, x, k, bias, bias_len, logits, idx, nullptr, status_dev, stream);
+}
+
+int nnq_linear_argmax_i64(const nnq_weight *w, const float *x, int64_t k, const float *bias, int64_t bias_len,
+                          float *logits, int64_t *idx, int32_t *status_dev, void *stream) {
+    return linear_argmax(w, x, k, bias, bias_len, logits, nullptr, idx, status_dev, stream);
 }
 
 // ---- MoE ---------------------------------------------------------------------------

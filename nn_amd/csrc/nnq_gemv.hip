@@ -1788,7 +1788,7 @@ __global__ __launch_bounds__(256) void dequant_q6k_kernel(const uint8_t *qs, con
     }
 }
 
-__global__ void argmax_final_kernel(const unsigned long long *partial, int64_t count, uint32_t *idx,
+__global__ void argmax_final_kernel(const unsigned long long *partial, int64_t count, uint32_t *idx, int64_t *idx64,
                                     int32_t *status) {
     __shared__ unsigned long long red[16];
     unsigned long long key = 0;
@@ -1813,7 +1813,9 @@ __global__ void argmax_final_kernel(const unsigned long long *partial, int64_t c
         unsigned long long k = 0;
         for (int i = 0; i < (int)(blockDim.x >> 6); i++) k = red[i] > k ? red[i] : k;
         const bool nan = (k == ~0ull);
-        *idx = nan ? 0u : 0xFFFFFFFFu - (uint32_t)(k & 0xFFFFFFFFu);
+        const uint32_t i = nan ? 0u : 0xFFFFFFFFu - (uint32_t)(k & 0xFFFFFFFFu);
+        if (idx) *idx = i;
+        if (idx64) *idx64 = (int64_t)i;
         if (status) *status = nan ? NNQ_ERR_NON_FINITE : NNQ_OK;
     }
 }
@@ -2139,9 +2141,10 @@ int launch_dequant(int fmt, const uint8_t *qs, const uint8_t *hdr, int64_t n, in
     return (int)hipGetLastError();
 }
 
-int launch_argmax_final(const unsigned long long *partial, int64_t count, uint32_t *idx, int32_t *status,
-                        void *stream) {
-    hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, partial, count, idx, status);
+int launch_argmax_final(const unsigned long long *partial, int64_t count, uint32_t *idx, int64_t *idx64,
+                        int32_t *status, void *stream) {
+    hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, partial, count, idx, idx64,
+                       status);
     return (int)hipGetLastError();
 }
 
@@ -2156,7 +2159,7 @@ int launch_argmax_reduce(const float *v, int64_t n, uint32_t *idx, int32_t *stat
     hipLaunchKernelGGL(argmax_partial_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, v, n, partial);
     int e = (int)hipGetLastError();
     if (e) return e;
-    return launch_argmax_final(partial, blocks, idx, status, stream);
+    return launch_argmax_final(partial, blocks, idx, nullptr, status, stream);
 }
 
 }  // namespace nnq

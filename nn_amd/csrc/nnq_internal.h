@@ -102,8 +102,9 @@ int launch_dequant(int fmt, const uint8_t *qs, const uint8_t *hdr, int64_t n, in
                    int64_t nblk, float *out, void *stream);
 int launch_argmax_reduce(const float *v, int64_t n, uint32_t *idx, int32_t *status, void *scratch,
                          size_t scratch_bytes, void *stream);
-int launch_argmax_final(const unsigned long long *partial, int64_t count, uint32_t *idx, int32_t *status,
-                        void *stream);
+// (the index to idx and / or idx64, whichever are given)
+int launch_argmax_final(const unsigned long long *partial, int64_t count, uint32_t *idx, int64_t *idx64,
+                        int32_t *status, void *stream);
 // MLP glue: h = silu(gate) * up from gu [m, 2 * inter] (gate | up halves, or with
 // interleaved8 the 8-gate-rows / 8-up-rows order of each 16 columns; clears *status when
 // given), and the non-finite output check (sets *status to NNQ_ERR_NON_FINITE)

@@ -154,12 +154,20 @@ def device_count() -> int:
     return c.value
 
 
+# The host side of a call is a good part of a small one (a decode linear's kernel takes 5 us), so
+# pointers pass as plain integers (the signatures declare them) and the stream's handle comes
+# from torch's raw accessor (0.1 us; a Stream object and its handle 2 us).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _device_input(t: torch.Tensor, what: str, device: Optional[int] = None) -> torch.Tensor:
@@ -175,6 +183,8 @@ def _device_input(t: torch.Tensor, what: str, device: Optional[int] = None) -> t
 
 def _side_input(t: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
     """A secondary operand (bias, router logits) as contiguous f32 on the device of `like`."""
+    if t.dtype is torch.float32 and t.device == like.device:
+        return t.contiguous()
     return t.to(device=like.device, dtype=torch.float32).contiguous()
 
 
@@ -283,7 +293,7 @@ def quantized_linear(input: torch.Tensor, weight: QuantizedWeight, bias: Optiona
             raise BiasMismatch(f"bias shape mismatch: expected [{n}], got {list(bias.shape)}")
         bias = _side_input(bias, x)
     out_dtype = out_dtype or torch.float32
-    y = torch.empty(tuple(x.shape[:-1]) + (n,), dtype=out_dtype, device=x.device)
+    y = x.new_empty((*x.shape[:-1], n), dtype=out_dtype)
     m = x.numel() // k
     _check(_lib.load().nnq_linear(weight.handle, _ptr(x), _DTYPE[x.dtype], m, k, _ptr(bias),
                                   n if bias is not None else 0, _ptr(y), _DTYPE[out_dtype], _stream(x)))
@@ -316,7 +326,7 @@ def argmax(logits: torch.Tensor) -> torch.Tensor:
         raise InvalidShape("argmax over a zero-length dimension")
     v = _device_input(logits, "logits").float().contiguous()
     idx = torch.empty(1, dtype=torch.int32, device=v.device)
-    st = torch.zeros(1, dtype=torch.int32, device=v.device)
+    st = torch.empty(1, dtype=torch.int32, device=v.device)  # written by the call
     _check(_lib.load().nnq_argmax_f32(_ptr(v), v.numel(), _ptr(idx), _ptr(st), _stream(v)))
     if int(st.item()) != 0:
         raise NonFiniteData("argmax/argmin input contains NaN")
@@ -334,14 +344,14 @@ def linear_argmax(x: torch.Tensor, weight: QuantizedWeight, bias: Optional[torch
         if bias.dim() != 1 or bias.shape[0] != n:
             raise BiasMismatch(f"bias shape mismatch: expected [{n}], got {list(bias.shape)}")
         bias = _side_input(bias, xv)
-    logits = torch.empty(n, dtype=torch.float32, device=xv.device)
-    idx = torch.empty(1, dtype=torch.int32, device=xv.device)
-    st = torch.zeros(1, dtype=torch.int32, device=xv.device)
-    _check(_lib.load().nnq_linear_argmax(weight.handle, _ptr(xv), k, _ptr(bias), n if bias is not None else 0,
-                                         _ptr(logits), _ptr(idx), _ptr(st), _stream(xv)))
+    logits = xv.new_empty(n)
+    idx = xv.new_empty((), dtype=torch.int64)
+    st = xv.new_empty(1, dtype=torch.int32) if check else None  # written by the call
+    _check(_lib.load().nnq_linear_argmax_i64(weight.handle, _ptr(xv), k, _ptr(bias), n if bias is not None else 0,
+                                             _ptr(logits), _ptr(idx), _ptr(st), _stream(xv)))
     if check and int(st.item()) != 0:
         raise NonFiniteData("argmax input contains NaN")
-    return logits, idx[0].to(torch.int64)
+    return logits, idx
 
 
 # ---------------------------------------------------------------------------------
@@ -449,8 +459,8 @@ class QuantizedMLP:
         xx = xx.reshape(-1, self.hidden).contiguous()
         m = xx.shape[0]
         od = out_dtype if out_dtype is not None else torch.float32
-        y = torch.empty((m, self.hidden), dtype=od, device=xx.device)
-        st = torch.zeros(1, dtype=torch.int32, device=xx.device)
+        y = xx.new_empty((m, self.hidden), dtype=od)
+        st = xx.new_empty(1, dtype=torch.int32) if check else None  # written by the call (m > 0)
         _check(_lib.load().nnq_mlp_forward(self._h, _ptr(xx), _DTYPE[xx.dtype], m, self.hidden, _ptr(y), _DTYPE[od],
                                            _ptr(st), _stream(xx)))
         if check and m > 0 and int(st.item()) != 0:
@@ -574,10 +584,10 @@ class QuantizedMoE:
         T = xx.shape[0]
         if top_k <= 0 or top_k > self.num_experts:
             raise InvalidShape(f"topk k={top_k} out of range for dim 1 (size {self.num_experts})")
-        y = torch.empty((T, self.hidden), dtype=torch.float32, device=xx.device)
-        ti = torch.empty((T, top_k), dtype=torch.int32, device=xx.device) if return_routing else None
-        tw = torch.empty((T, top_k), dtype=torch.float32, device=xx.device) if return_routing else None
-        st = torch.zeros(1, dtype=torch.int32, device=xx.device)
+        y = xx.new_empty((T, self.hidden), dtype=torch.float32)
+        ti = xx.new_empty((T, top_k), dtype=torch.int32) if return_routing else None
+        tw = xx.new_empty((T, top_k), dtype=torch.float32) if return_routing else None
+        st = xx.new_empty(1, dtype=torch.int32) if check else None  # written by the call (T > 0)
         _check(_lib.load().nnq_moe_block_forward(self._h, self._router, _ptr(xx), _DTYPE[xx.dtype], T, int(top_k),
                                                  float(swiglu_limit), _ptr(y), _ptr(ti), _ptr(tw), _ptr(st),
                                                  _stream(xx)))
@@ -597,9 +607,9 @@ class QuantizedMoE:
         if top_k <= 0 or top_k > self.num_experts:
             raise InvalidShape(f"topk k={top_k} out of range for dim 1 (size {self.num_experts})")
         lg = _side_input(router_logits, xx)
-        y = torch.empty((T, self.hidden), dtype=torch.float32, device=xx.device)
-        ti = torch.empty((T, top_k), dtype=torch.int32, device=xx.device) if return_routing else None
-        tw = torch.empty((T, top_k), dtype=torch.float32, device=xx.device) if return_routing else None
+        y = xx.new_empty((T, self.hidden), dtype=torch.float32)
+        ti = xx.new_empty((T, top_k), dtype=torch.int32) if return_routing else None
+        tw = xx.new_empty((T, top_k), dtype=torch.float32) if return_routing else None
         _check(_lib.load().nnq_moe_forward(self._h, _ptr(xx), _DTYPE[xx.dtype], T, _ptr(lg), int(top_k),
                                            float(swiglu_limit), _ptr(y), _ptr(ti), _ptr(tw), _stream(xx)))
         if return_routing:
