@@ -4,7 +4,7 @@
 // crates/nn-core/src/dyn_tensor/ops/matmul.rs:37-38).
 //
 // Workgroup: eight waves stacked along M, 256 rows x NT * 16 columns (NT = 6: 96 columns, one
-// workgroup per CU at 512 x 12288; NT = 4 with the K range split in two at 512 x 4096).  Each
+// workgroup per CU at 512 x 12288; NT = 8 with the K range split in four at 512 x 4096).  Each
 // wave owns 32 rows (two 16-row MFMA tiles) across all NT column tiles, so a B fragment read
 // from LDS serves two MFMAs and an A fragment NT of them; the activation is the operand with
 // the higher reuse and is read from L2 straight into registers, the weight is the one shared
@@ -50,7 +50,7 @@ template <int NT>
 struct Wide {
     static constexpr int BN = NT * 16;
     static constexpr int BFRAG = NT * 8 * 1024;  // dequantized B of a super-block: tiles x steps x 1 KB
-    static constexpr int D_OFF = BFRAG;          // d of each column (f32)
+    static constexpr int D_OFF = BFRAG;          // d of each column in the totals' unit (f32)
     static constexpr int BUF = D_OFF + NT * 16 * 4;
     // min-term B operands (tiles x 1 KB) in a ring of three: the MFMAs that use a
     // super-block's run in the first step of the next one
@@ -159,8 +159,9 @@ __device__ __forceinline__ uint32_t bload1(__amdgpu_buffer_rsrc_t r, int voff, i
 template <int NT, int P>
 __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     using C = Wide<NT>;
-    constexpr int PPT = C::PPT, PD = P == 1 ? 3 : 2;  // A-fragment prefetch distance in 32-k steps
-    constexpr int RING = P == 1 ? PD + 1 : PD + 2;    // (a divisor of the 8 steps)
+    constexpr int PPT = C::PPT, PD = NT == 8 ? 1 : P == 1 ? 3 : 2;  // A-fragment prefetch distance in 32-k steps
+    constexpr int RING = PD == 1 ? 2 : 4;                           // (a divisor of the 8 steps)
+    constexpr int BH = NT == 8 ? 4 : NT;                            // B fragments held at a time
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -199,25 +200,36 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
     const int qoff = ph * 1024 + (16 * pgp + c16) * 16, hoff = c16 * 16;
     const int xoff = (lane >> 5) * 256 + c16 * 16;
     const int tw = __builtin_amdgcn_readfirstlane(tid >> 7);  // tile of this thread's first piece
-    // per column: 2^16 or 2^-8 times s_n, what brings the partial sums to the totals' unit (s_n a normal power of two), and the epilogue's
-    // factors, loaded now: 2^8 / s_n and the bias per column, 2^-s_row per row
     const float *srow = reinterpret_cast<const float *>(a.aux + (size_t)a.ntile * nblk * 512);
-    float f1[NT], f2[NT], bc[NT], rb[MT][4];
+    // 2^16 or 2^-8 times s_n of the columns whose d this thread stores (one per piece): what brings
+    // the partial sums to the totals' unit (s_n a normal power of two)
+    float f1[PPT];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const uint32_t eb = __float_as_uint(srow[(size_t)(t0 + nt) * 16 + c16]) >> 23;
-        f1[nt] = __uint_as_float((P == 1 ? eb + 16u : eb - 8u) << 23);
-        f2[nt] = __uint_as_float((262u - eb) << 23);
-        bc[nt] = (a.bias && a.ks == 1) ? a.bias[(int64_t)(t0 + nt) * 16 + c16] : 0.0f;
+    for (int j = 0; j < PPT; j++) {
+        const uint32_t eb = __float_as_uint(srow[(size_t)min(t0 + tw + 4 * j, a.ntile - 1) * 16 + c16]) >> 23;
+        f1[j] = __uint_as_float((P == 1 ? eb + 16u : eb - 8u) << 23);
     }
+    // the epilogue's factors: 2^8 / s_n and the bias per column, 2^-s_row per row.  Loaded now, or
+    // with eight column tiles (whose loop needs the registers) before the last min term.
+    constexpr bool LATE = NT == 8;
+    float f2[NT], bc[NT], rb[MT][4];
+    auto load_factors = [&]() {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        // rows 4G .. 4G + 3 of the tile: one 16-byte load (the rowback plane is padded to 16 rows)
-        const floatx4 v = *reinterpret_cast<const floatx4 *>(
-            a.rowback + min(rt * BM + wv * 32 + mt * 16, a.nrg * 16 - 16) + 4 * G);
+        for (int nt = 0; nt < NT; nt++) {
+            const uint32_t eb = __float_as_uint(srow[(size_t)(t0 + nt) * 16 + c16]) >> 23;
+            f2[nt] = __uint_as_float((262u - eb) << 23);
+            bc[nt] = (a.bias && a.ks == 1) ? a.bias[(int64_t)(t0 + nt) * 16 + c16] : 0.0f;
+        }
 #pragma unroll
-        for (int e = 0; e < 4; e++) rb[mt][e] = v[e];
-    }
+        for (int mt = 0; mt < MT; mt++) {
+            // rows 4G .. 4G + 3 of the tile: one 16-byte load (the rowback plane is padded to 16 rows)
+            const floatx4 v = *reinterpret_cast<const floatx4 *>(
+                a.rowback + min(rt * BM + wv * 32 + mt * 16, a.nrg * 16 - 16) + 4 * G);
+#pragma unroll
+            for (int e = 0; e < 4; e++) rb[mt][e] = v[e];
+        }
+    };
+    if constexpr (!LATE) load_factors();
 
     // the next super-block's raw operands (issued one super-block ahead)
     u32x4 raw[PPT], hd[PPT];
@@ -247,7 +259,7 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
 #pragma unroll
             for (int hh = 0; hh < 2; hh++)
                 *reinterpret_cast<u32x4 *>(buf + ((t * 8 + 2 * pgp + hh) * 64 + 16 * (2 * ph + g) + c16) * 16) = o[g][hh];
-        if (pgp == 0 && ph == 0) *reinterpret_cast<float *>(buf + C::D_OFF + (t * 16 + c16) * 4) = f16_to_f32(hd[j][0] & 0xFFFFu);
+        if (pgp == 0 && ph == 0) *reinterpret_cast<float *>(buf + C::D_OFF + (t * 16 + c16) * 4) = f16_to_f32(hd[j][0] & 0xFFFFu) * f1[j];
     };
 
     floatx4 tot[MT][NT], part[MT][NT];
@@ -302,31 +314,37 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
                 for (int pl = 0; pl < P; pl++)
                     af[(s + PD) % RING][mt][pl] = bload4(ra[mt][pl], loff, (sb * 8 + s + PD) * 1024);
             __builtin_amdgcn_sched_barrier(0);
-            u32x4 bf[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) bf[nt] = *reinterpret_cast<const u32x4 *>(cur + ((nt * 8 + s) * 64 + lane) * 16);
             if (s == 0 && sb > 0) min_term(sb - 1, xsp_prev);
             if (s == 6) {
-                // the super-block's factor d per column (f1 folded in)
+                // the super-block's factor d per column (with f1)
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++)
-                    dn[nt] = *reinterpret_cast<const float *>(cur + C::D_OFF + (nt * 16 + c16) * 4) * f1[nt];
+                    dn[nt] = *reinterpret_cast<const float *>(cur + C::D_OFF + (nt * 16 + c16) * 4);
             }
 #pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
+            for (int n0 = 0; n0 < NT; n0 += BH) {
+                u32x4 bf[BH];
 #pragma unroll
-                for (int pl = P - 1; pl >= 0; pl--)
+                for (int j = 0; j < BH; j++)
+                    bf[j] = *reinterpret_cast<const u32x4 *>(cur + (((n0 + j) * 8 + s) * 64 + lane) * 16);
 #pragma unroll
-                    for (int mt = 0; mt < MT; mt++)
-                        part[mt][nt] = mfma16x16x32_f16(af[s % RING][mt][pl], bf[nt],
-                                                        s == 0 && pl == P - 1 ? floatx4{0.f, 0.f, 0.f, 0.f}
-                                                                              : part[mt][nt]);
-                if (s == 7) {
+                for (int j = 0; j < BH; j++) {
+                    const int nt = n0 + j;
 #pragma unroll
-                    for (int mt = 0; mt < MT; mt++)
+                    for (int pl = P - 1; pl >= 0; pl--)
 #pragma unroll
-                        for (int e = 0; e < 4; e++) tot[mt][nt][e] += dn[nt] * part[mt][nt][e];
+                        for (int mt = 0; mt < MT; mt++)
+                            part[mt][nt] = mfma16x16x32_f16(af[s % RING][mt][pl], bf[j],
+                                                            s == 0 && pl == P - 1 ? floatx4{0.f, 0.f, 0.f, 0.f}
+                                                                                  : part[mt][nt]);
+                    if (s == 7) {
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) tot[mt][nt][e] += dn[nt] * part[mt][nt][e];
+                    }
                 }
+                if constexpr (NT == 8) __builtin_amdgcn_sched_barrier(0);
             }
             // the next super-block's operands into the other buffer (read by nobody since
             // the barrier that ended the previous super-block), one piece every other step;
@@ -342,6 +360,7 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q4k_wide_kernel(WideArgs a) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (LATE) load_factors();
     min_term(nsb - 1, xsp_prev);
     // every wave has read the aux ring before the output tile (f32: over the ring) is written
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -675,21 +694,25 @@ __global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const void *xv, in
 // padding: f32 x, 100 x 4096 x 12288 109 us against the ring's 51), whole 16-row weight tiles
 // and a 16-byte aligned output (the epilogue writes 16-byte row chunks), K <= 4096 * 3 (the
 // staging keeps the row in one workgroup's registers and its sub-block sums in LDS), and at
-// least 128 workgroups.  Column tiles per workgroup (6 or 4) and K split (1 to 4 equal parts
+// least 128 workgroups.  Column tiles per workgroup (6, 4 or 8) and K split (1 to 4 equal parts
 // of whole super-blocks) are the ones with the least estimated time: rounds of workgroups over
-// the CUs, times super-blocks, times the measured time of one (us, 6 and 4 tiles: bf16 x 3.8
-// and 3.0, f32 x 6.1 and 5.2), plus the slabs' write, read and launch.  512 rows of f32 x take
-// 106 us at 12288 x 4096 (6 tiles; the ring kernel over two planes 153) and 134 at 4096 x 12288
-// (4 tiles, K in two; 155); 203 rows at 12288 x 4096 take 6 tiles and K in two (256 workgroups).
+// the CUs, times super-blocks, times the measured time of one (us, 6, 4 and 8 tiles: bf16 x
+// 3.8, 3.0 and 5.0, f32 x 6.2, 5.2 and 7.8: more tiles read each A fragment less often), plus
+// the slabs' write, read and launch.  512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles;
+// the ring kernel over two planes 153) and 115 at 4096 x 12288 (8 tiles, K in four; 4 tiles
+// and K in two 134, ring 155), of bf16 x there 77 (4 tiles 83); 203 rows of f32 x at 12288 x
+// 4096 take 6 tiles and K in two (256 workgroups).
+// With random x these rates are the chip's power limit for f16 products: a library f16 GEMM
+// of 512 x 12288 x 4096 takes 58 us (44 with x = 0), this kernel 66 with its staging (60).
 // Returns the column tiles per workgroup (0: the ring kernel takes the shape) and the K split.
 int gemm_wide_plan(const GemmArgs &a, int *ks) {
     if (a.blk || a.m <= 128 || a.k > 4096 * 3 || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
     const int64_t nrt = (a.m + BM - 1) / BM;
-    const float sb_us[2][2] = {{3.8f, 3.0f}, {6.1f, 5.2f}};
+    const float sb_us[2][3] = {{3.8f, 3.0f, 5.0f}, {6.2f, 5.2f, 7.8f}};
     float best = 0.0f;
     int nt = 0;
-    for (int i = 0; i < 2; i++) {
-        const int c = i == 0 ? 6 : 4;
+    for (int i = 0; i < 3; i++) {
+        const int c = i == 0 ? 6 : i == 1 ? 4 : 8;
         if (a.ntile % c) continue;
         for (int split = 1; split <= 4; split++) {
             const int64_t wg = nrt * (a.ntile / c) * split;
@@ -836,9 +859,9 @@ int launch_gemm_wide(const GemmArgs &a, const GemmScratch &sc, void *stream) {
         return launch_skinny_cfg<3, 2, 8>(w, st);  // the plan: 17 to 32 rows, three tiles, eight waves
     }
     if (a.x_bf16)
-        e = nt == 6 ? launch_wide_nt<6, 1>(w, st) : launch_wide_nt<4, 1>(w, st);
+        e = nt == 8 ? launch_wide_nt<8, 1>(w, st) : nt == 6 ? launch_wide_nt<6, 1>(w, st) : launch_wide_nt<4, 1>(w, st);
     else
-        e = nt == 6 ? launch_wide_nt<6, 2>(w, st) : launch_wide_nt<4, 2>(w, st);
+        e = nt == 8 ? launch_wide_nt<8, 2>(w, st) : nt == 6 ? launch_wide_nt<6, 2>(w, st) : launch_wide_nt<4, 2>(w, st);
     if (e || ks == 1) return e;
     return launch_gemm_finalize(sc.ysplit, ks, a.bias, a.y, a.y_bf16, a.m, a.n, stream);
 }

@@ -69,17 +69,20 @@ def test_wide_row_scales(O, dev):
 
 
 # f32 activations (hi + lo planes) on the wide kernel: one row past its lower limit, ragged row
-# tiles, both column-tile widths, K split two to four ways and not at all, K of the staging's
-# limit.  Bar: max |error| <= 2e-5 of the output's rms: f32 sums over K <= 12288 of products
+# tiles, the three column-tile widths (the last three shapes: eight tiles, also for bf16), K split
+# two to four ways and not at all, K of the staging's limit.  Bar: max |error| <= 2e-5 of the output's rms: f32 sums over K <= 12288 of products
 # that keep 22 bits of x (2.3e-6 measured at 512 x 4096 x 12288).
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(129, 3072, 1024), (203, 12288, 512), (300, 6144, 2048), (513, 4096, 1280),
-                                   (256, 1024, 12288), (700, 1920, 768)])
-def test_wide_f32_activations(dev, m, n, k):
+                                   (256, 2048, 12288), (700, 1920, 768), (512, 4096, 2048), (1100, 4096, 512),
+                                   (1000, 2048, 2560)])
+def test_wide_activations(dev, m, n, k, xdt):
     import nn_amd
     w = make_weight("q4_k", nn_amd.quantize_q4_k(nn_amd.synth_normal(m, 1, (n, k), 0.02)), n, k)
     x = torch.from_numpy(nn_amd.synth_normal(m, 2, (m, k), 1.0)).to(dev)
     x[5] *= 1e-20
     x[7] = 0.0
+    x = x.to(xdt)
     bias = torch.from_numpy(nn_amd.synth_normal(m, 3, (n,), 0.5)).to(dev)
     y = nn_amd.quantized_linear(x, w, bias)
     assert torch.equal(y, nn_amd.quantized_linear(x, w, bias)), "repeated calls must agree bit for bit"
