@@ -63,6 +63,12 @@ GemmScratch gemm_carve(void *base, const GemmArgs &a, size_t *bytes) {
         if (bytes) *bytes = off;
         return s;
     }
+    if (gemm_wide6_plan(a)) {
+        GemmScratch s{};
+        const size_t off = gemm_wide6_scratch(a, &s, b);
+        if (bytes) *bytes = off;
+        return s;
+    }
     size_t off = 0;
     GemmScratch s;
     s.xh = reinterpret_cast<uint16_t *>(b + off);

@@ -195,6 +195,10 @@ int launch_stage_wide(const void *x, int x_bf16, int64_t m, int64_t k, void *xa,
 int gemm_wide8_plan(const GemmArgs &a, int *ks);
 size_t gemm_wide8_scratch(const GemmArgs &a, GemmScratch *s, uint8_t *base);
 int launch_gemm_wide8(const GemmArgs &a, const GemmScratch &sc, void *stream);
+// Q6_K wide kernel (nnq_gemm_wide6.hip): its K split (0: not its shape), scratch and launch
+int gemm_wide6_plan(const GemmArgs &a);
+size_t gemm_wide6_scratch(const GemmArgs &a, GemmScratch *s, uint8_t *base);
+int launch_gemm_wide6(const GemmArgs &a, const GemmScratch &sc, void *stream);
 // split-K result: ks f32 slabs [m][n] summed in order, plus the bias, to f32 or bf16 (n % 4 == 0)
 int launch_gemm_finalize(const float *ys, int ks, const float *bias, void *y, int y_bf16, int64_t m, int64_t n,
                          void *stream);

@@ -173,3 +173,30 @@ def test_gemm_q80_wide(O, dev, m, n, k):
     # the bf16 output is the f32 result rounded once
     yb = nn_amd.quantized_linear(xt, w, bias, out_dtype=torch.bfloat16)
     assert torch.equal(yb, y.to(torch.bfloat16)), "bf16 output is not the f32 result rounded once"
+
+
+# The wide Q6_K kernel (bf16 x, more than 128 rows, whole groups of 8 weight tiles): one row past
+# its lower limit, ragged row tiles, K not split and split 2, 3, 4, 7 and 8 ways, the fewest
+# super-blocks of a part, every sign of the int8 scales (and one shape it leaves to the block kernel).  Bar: products are exact in f32, so max |error| <= 1e-5 of
+# the output's rms (f32 sums over K <= 12288; 9e-7 measured at 512 x 4096 x 12288).
+@pytest.mark.parametrize("m,n,k", [(129, 24576, 512), (385, 8192, 1536), (200, 8192, 1536), (300, 4096, 2048),
+                                   (517, 1536, 3584), (200, 4096, 6144), (512, 12288, 512), (1025, 4096, 1536)])
+def test_wide_q6k(m, n, k):
+    import nn_amd
+    nn_amd.init(0)
+    b = nn_amd.quantize_q6_k(nn_amd.synth_normal(m, 1, (n, k), 0.02)).reshape(-1, 210).copy()
+    b[::3, 192:208] = (256 - b[::3, 192:208].astype(np.int32)).astype(np.uint8)  # negated scales
+    b[1::5, 192] = 128  # -128
+    w = nn_amd.QuantizedWeight.from_quantized(b.ravel(), nn_amd.QuantType.Q6_K, (n, k), layout=nn_amd.Layout.NN_GGUF)
+    x = torch.from_numpy(nn_amd.synth_normal(m, 2, (m, k), 1.0)).cuda()
+    x[5] *= 1e-20
+    x[7] = 0.0
+    x = x.to(torch.bfloat16)
+    bias = torch.from_numpy(nn_amd.synth_normal(m, 3, (n,), 0.5)).cuda()
+    y = nn_amd.quantized_linear(x, w, bias)
+    assert torch.equal(y, nn_amd.quantized_linear(x, w, bias)), "repeated calls must agree bit for bit"
+    ref = x.double() @ w.dequantize().double().t() + bias.double()
+    err = ((y.double() - ref).abs().amax(1) / ref.pow(2).mean(1).sqrt()).max().item()
+    assert err <= 1e-5, f"{m}x{n}x{k}: {err:.2e} of the row's rms"
+    yb = nn_amd.quantized_linear(x, w, bias, out_dtype=torch.bfloat16)
+    assert torch.equal(yb, y.to(torch.bfloat16)), "bf16 output: the f32 result rounded once"
