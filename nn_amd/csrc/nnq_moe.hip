@@ -442,222 +442,60 @@ __global__ __launch_bounds__(256) void moe_route_any_kernel(const float *logits,
     }
 }
 
-// One workgroup of 1024 threads, one token per thread per chunk of 1024 tokens.  For
-// each expert a ballot gives every token its rank among the wave's tokens that chose
-// the expert; per-wave counts in LDS turn that into the rank over all earlier tokens.
-// Expert e's rows are then its tokens in ascending order (stable by token, the order
-// moe_forward's grouping loop builds, crates/nn-gptoss/src/quantized_model.rs:157-169).
-// Experts go in groups of 256 (the per-wave count table); the running per-expert
-// totals live in dynamic shared memory (E ints).
-template <int k>
-__global__ __launch_bounds__(1024) void moe_permute_kernel(const uint32_t *ti, int64_t T, int E, int32_t *off,
-                                                           int32_t *stok, int32_t *pos) {
-    __shared__ int32_t wcnt[16][256];
-    extern __shared__ int32_t base[];  // [E]
+// Batches over 1024 tokens: one workgroup per expert (in place of one workgroup for all, whose
+// ballots per expert and chunk took 22 us at 2048 tokens of 32 experts, 8 us here).  It reads
+// every assignment: those to lower experts give the expert's first row, its own tokens are
+// ranked by ballots per wave and counts per chunk of 1024 tokens, and collected in LDS, since
+// their rows are known only at the end.  Expert e's rows are then its tokens in ascending order
+// (stable by token, the order moe_forward's grouping loop builds,
+// crates/nn-gptoss/src/quantized_model.rs:157-169).
+constexpr int kMoePermThreads = 1024;
+__global__ __launch_bounds__(kMoePermThreads) void moe_permute_kernel(const uint32_t *ti, int64_t T, int E, int k,
+                                                                      int32_t *off, int32_t *stok, int32_t *pos) {
+    constexpr int W = kMoePermThreads / 64;
+    __shared__ int32_t wc[2][W], wb[W];
+    extern __shared__ int32_t tok[];  // [T] the expert's tokens
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const uint32_t e = blockIdx.x;
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-    for (int e = tid; e < E; e += 1024) base[e] = 0;
-    __syncthreads();
-    // with one chunk (T <= 1024) each thread keeps its token's experts and ranks in
-    // registers for the final scatter; longer batches pass the ranks through pos
-    const bool one_chunk = T <= 1024;
-    uint32_t ex[k];
-    int32_t myrank[k];
-    for (int64_t t0 = 0; t0 < T; t0 += 1024) {
+    int below = 0, ne = 0, par = 0;
+    for (int64_t t0 = 0; t0 < T; t0 += kMoePermThreads, par ^= 1) {
         const int64_t t = t0 + tid;
-#pragma unroll
-        for (int s = 0; s < k; s++) ex[s] = t < T ? ti[t * k + s] : 0xFFFFFFFFu;
-        for (int g0 = 0; g0 < E; g0 += 256) {
-            const int ge = min(256, E - g0);
-            int32_t rk[k];
-#pragma unroll
-            for (int s = 0; s < k; s++) rk[s] = 0;
-            // waves past the batch only publish zero counts (a short batch leaves most of
-            // the 16 waves idle: 256 tokens use 4)
-            const bool live = t0 + (int64_t)wv * 64 < T;  // wave-uniform
-            for (int e = 0; e < ge; e++) {
-                if (!live) {
-                    if (lane == 0) wcnt[wv][e] = 0;
-                    continue;
-                }
-                const uint32_t ee = (uint32_t)(g0 + e);
-                bool hit = false;
-#pragma unroll
-                for (int s = 0; s < k; s++) hit |= ex[s] == ee;
-                const uint64_t m = __ballot(hit);
-                const int32_t r = __popcll(m & lt);
-#pragma unroll
-                for (int s = 0; s < k; s++)
-                    if (ex[s] == ee) rk[s] = r;
-                if (lane == 0) wcnt[wv][e] = __popcll(m);
+        bool hit = false;  // a token routes to an expert at most once
+        if (t < T)
+            for (int q = 0; q < k; q++) {
+                const uint32_t x = ti[t * k + q];
+                below += x < e ? 1 : 0;
+                hit |= x == e;
             }
-            __syncthreads();
-            // per expert (one per thread): wcnt[w][e] becomes the count of earlier tokens,
-            // base plus the waves before w (the 16 loads independent of each other)
-            for (int e = tid; e < ge; e += 1024) {
-                int32_t c[16];
+        const uint64_t m = __ballot(hit);
+        if (lane == 0) wc[par][wv] = __popcll(m);
+        __syncthreads();  // the counts alternate between two rows, so one barrier per chunk
+        int before = ne, total = 0;
 #pragma unroll
-                for (int w = 0; w < 16; w++) c[w] = wcnt[w][e];
-                int32_t run = base[g0 + e];
-#pragma unroll
-                for (int w = 0; w < 16; w++) {
-                    wcnt[w][e] = run;
-                    run += c[w];
-                }
-                base[g0 + e] = run;
-            }
-            __syncthreads();
-            if (t < T)
-#pragma unroll
-                for (int s = 0; s < k; s++)
-                    if (ex[s] >= (uint32_t)g0 && ex[s] < (uint32_t)(g0 + ge)) {
-                        const int32_t r = wcnt[wv][ex[s] - g0] + rk[s];  // rank within the expert; offset below
-                        if (one_chunk)
-                            myrank[s] = r;
-                        else
-                            pos[t * k + s] = r;
-                    }
-            __syncthreads();  // wcnt is rewritten by the next group / chunk
+        for (int w = 0; w < W; w++) {
+            const int c = wc[par][w];
+            before += w < wv ? c : 0;
+            total += c;
         }
+        if (hit) tok[before + __popcll(m & lt)] = (int32_t)t;
+        ne += total;
     }
-    if (tid < 64) {
-        // exclusive scan of the expert counts, 256 at a time: lane l holds experts
-        // c0 + 4l .. c0 + 4l + 3, the carry is the total of the earlier groups
-        int32_t carry = 0;
-        for (int c0 = 0; c0 < E; c0 += 256) {
-            int32_t c[4], sum = 0;
+    below = wave_sum_i32(below);
+    if (lane == 0) wb[wv] = below;
+    __syncthreads();  // also publishes tok
+    int32_t r0 = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int e = c0 + 4 * tid + j;
-                c[j] = e < E ? base[e] : 0;
-                sum += c[j];
-            }
-            int32_t before = sum;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int32_t v = __shfl_up(before, o, 64);
-                if (tid >= o) before += v;
-            }
-            const int32_t total = __shfl(before, 63, 64);
-            before += carry - sum;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int e = c0 + 4 * tid + j;
-                if (e < E) {
-                    base[e] = before;
-                    off[e] = before;
-                }
-                before += c[j];
-            }
-            carry += total;
-        }
-        if (tid == 0) off[E] = carry;  // the total
+    for (int w = 0; w < W; w++) r0 += wb[w];
+    if (tid == 0) {
+        off[e] = r0;
+        if ((int)e == E - 1) off[E] = (int32_t)(T * k);
     }
-    __syncthreads();
-    if (one_chunk) {
-        if (tid < T)
-#pragma unroll
-            for (int s = 0; s < k; s++) {
-                const int32_t p = myrank[s] + base[ex[s]];
-                pos[tid * k + s] = p;
-                stok[p] = tid;
-            }
-        return;
-    }
-    for (int64_t i = tid; i < T * k; i += 1024) {
-        const int32_t p = pos[i] + base[ti[i]];
-        pos[i] = p;
-        stok[p] = (int32_t)(i / k);
-    }
-}
-
-// moe_permute_kernel for any k (k > 8): the token's experts are read from ti inside the
-// expert loop instead of registers, and the ranks go through pos.
-__global__ __launch_bounds__(1024) void moe_permute_any_kernel(const uint32_t *ti, int64_t T, int E, int k,
-                                                               int32_t *off, int32_t *stok, int32_t *pos) {
-    __shared__ int32_t wcnt[16][256];
-    extern __shared__ int32_t base[];  // [E]
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-    for (int e = tid; e < E; e += 1024) base[e] = 0;
-    __syncthreads();
-    for (int64_t t0 = 0; t0 < T; t0 += 1024) {
-        const int64_t t = t0 + tid;
-        for (int g0 = 0; g0 < E; g0 += 256) {
-            const int ge = min(256, E - g0);
-            const bool live = t0 + (int64_t)wv * 64 < T;  // wave-uniform
-            for (int e = 0; e < ge; e++) {
-                if (!live) {
-                    if (lane == 0) wcnt[wv][e] = 0;
-                    continue;
-                }
-                const uint32_t ee = (uint32_t)(g0 + e);
-                int sh = -1;  // the token routes to an expert at most once
-                if (t < T)
-                    for (int s = 0; s < k; s++)
-                        if (ti[t * k + s] == ee) sh = s;
-                const uint64_t m = __ballot(sh >= 0);
-                if (sh >= 0) pos[t * k + sh] = __popcll(m & lt);  // rank within the wave
-                if (lane == 0) wcnt[wv][e] = __popcll(m);
-            }
-            __syncthreads();
-            for (int e = tid; e < ge; e += 1024) {
-                int32_t c[16];
-#pragma unroll
-                for (int w = 0; w < 16; w++) c[w] = wcnt[w][e];
-                int32_t run = base[g0 + e];
-#pragma unroll
-                for (int w = 0; w < 16; w++) {
-                    wcnt[w][e] = run;
-                    run += c[w];
-                }
-                base[g0 + e] = run;
-            }
-            __syncthreads();
-            if (t < T)
-                for (int s = 0; s < k; s++) {
-                    const uint32_t ex = ti[t * k + s];
-                    if (ex >= (uint32_t)g0 && ex < (uint32_t)(g0 + ge)) pos[t * k + s] += wcnt[wv][ex - g0];
-                }
-            __syncthreads();
-        }
-    }
-    if (tid < 64) {
-        int32_t carry = 0;
-        for (int c0 = 0; c0 < E; c0 += 256) {
-            int32_t c[4], sum = 0;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int e = c0 + 4 * tid + j;
-                c[j] = e < E ? base[e] : 0;
-                sum += c[j];
-            }
-            int32_t before = sum;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int32_t v = __shfl_up(before, o, 64);
-                if (tid >= o) before += v;
-            }
-            const int32_t total = __shfl(before, 63, 64);
-            before += carry - sum;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int e = c0 + 4 * tid + j;
-                if (e < E) {
-                    base[e] = before;
-                    off[e] = before;
-                }
-                before += c[j];
-            }
-            carry += total;
-        }
-        if (tid == 0) off[E] = carry;
-    }
-    __syncthreads();
-    for (int64_t i = tid; i < T * k; i += 1024) {
-        const int32_t p = pos[i] + base[ti[i]];
-        pos[i] = p;
-        stok[p] = (int32_t)(i / k);
+    for (int i = tid; i < ne; i += kMoePermThreads) {
+        const int64_t t = tok[i];
+        stok[r0 + i] = (int32_t)t;
+        for (int q = 0; q < k; q++)
+            if (ti[t * k + q] == e) pos[t * k + q] = r0 + i;
     }
 }
 
@@ -844,7 +682,10 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
     // Workgroup ids go round-robin over the 8 XCDs; when the count allows, XCD x gets a
     // contiguous run of (expert, group) items, i.e. whole experts, so an expert's
     // activation rows are read into one XCD's L2 only.
-    const int nwg = (int)gridDim.x, bid = (int)blockIdx.x;
+    // The grid holds `slots` such sets: a workgroup takes every slots-th 64-row pass of its group,
+    // so that the passes of experts with many rows spread over the chip.
+    const int nwg = (int)d.E * kMoeGroups, bid = (int)blockIdx.x % nwg, slot0 = (int)blockIdx.x / nwg;
+    const int slots = (int)gridDim.x / nwg;
     const int item = (nwg % 8 == 0) ? (bid % 8) * (nwg / 8) + bid / 8 : bid;
     const int64_t e = item / kMoeGroups, g = item % kMoeGroups;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -853,7 +694,7 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
     int32_t *tok_s = reinterpret_cast<int32_t *>(smem + C::RING + (SL ? (size_t)kMoeWaves * NBW * KBP * 32 : 0));
     int32_t r0, ne;
     if (GU && run.perm) {
-        // moe_permute_kernel's result for this expert: r0 = the assignments to lower
+        // as moe_permute_kernel: r0 = the assignments to lower
         // experts, the rows = its tokens in ascending order (a token routes to an expert
         // at most once), counted per wave and ordered by lane rank
         int32_t *wc = tok_s + kMoeInPermT;  // [2][kMoeWaves]
@@ -890,7 +731,7 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
         // the same in every lane: scalar registers for the epilogue's uniform addressing
         r0 = __builtin_amdgcn_readfirstlane(r0);
         ne = __builtin_amdgcn_readfirstlane(ne);
-        if (g == 0) {
+        if (g == 0 && slot0 == 0) {
             // for the down and combine launches: the expert's first row, the total, and
             // each assignment's row
             if (tid == 0) {
@@ -913,7 +754,7 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
     const int nch = (int)(KB / CKB);  // K / 32 is a multiple of CKB (the host picks CKB)
     unsigned char *scl = smem + C::RING + (size_t)wv * NBW * KBP * 32;  // this wave's scales (SL)
 
-    for (int32_t m0 = 0; m0 < ne; m0 += 64) {
+    for (int32_t m0 = slot0 * 64; m0 < ne; m0 += slots * 64) {
         const int mtn = (ne - m0) >= 64 ? 4 : (ne - m0 + 15) / 16;  // live row tiles
         // copy sources of this pass: granule c -> (plane, row, slot); chunk ch at + ch * CKB * 32 k.
         // A 32-bit byte offset per lane from one uniform base (the planes of an activation
@@ -1615,8 +1456,15 @@ static int launch_stream_t(const MoeDev &d, const MoeScratch &sc, const MoeRun &
         if (e != hipSuccess) return (int)e;
         attr_set = true;
     }
-    hipLaunchKernelGGL((moe_stream_kernel<P, GU, CKB, SL>), dim3((unsigned)(d.E * kMoeGroups)), dim3(kMoeWaves * 64),
-                       lds, st, d, sc, run);
+    // One slot while an expert has up to 64 rows on average (a slot without a pass still starts a
+    // workgroup), then enough for half again the average, at most 4 (more cost what they give:
+    // 2048 tokens of 32 experts of 2048 x 2048 576 us with 1, 511 with 2, 498 with 4, 527 with
+    // 5).  400 tokens on 16 experts 291 -> 174 us, 1000 f32 tokens on 8 of 2880 x 1440 566 ->
+    // 232; 32 experts of 2880 x 2880, whose one set already fills the chip, within 1%.
+    const int64_t avg = run.A / d.E;
+    const int64_t slots = avg <= 64 ? 1 : std::min<int64_t>(4, (avg + avg / 2 + 63) / 64);
+    hipLaunchKernelGGL((moe_stream_kernel<P, GU, CKB, SL>), dim3((unsigned)(d.E * kMoeGroups * slots)),
+                       dim3(kMoeWaves * 64), lds, st, d, sc, run);
     return (int)hipGetLastError();
 }
 
@@ -1685,18 +1533,17 @@ int launch_moe(const MoeDev &d, const void *x, int x_bf16, int64_t T, const floa
         hipLaunchKernelGGL(moe_route_any_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256),
                            (size_t)4 * (d.E + (k > 8 ? k : 0)) * 4, st, logits, nsplit, bias, T, (int)d.E, k, sc.ti,
                            sc.tw, topk_idx, topk_w);
-    if (!run.perm) switch (k) {
-#define NNQ_PERM(K)                                                                                              \
-    case K:                                                                                                      \
-        hipLaunchKernelGGL(moe_permute_kernel<K>, dim3(1), dim3(1024), (size_t)d.E * 4, st, sc.ti, T, (int)d.E, sc.off, \
-                           sc.stok, sc.pos);                                                                     \
-        break;
-        NNQ_PERM(1) NNQ_PERM(2) NNQ_PERM(3) NNQ_PERM(4) NNQ_PERM(5) NNQ_PERM(6) NNQ_PERM(7) NNQ_PERM(8)
-#undef NNQ_PERM
-    default:
-        hipLaunchKernelGGL(moe_permute_any_kernel, dim3(1), dim3(1024), (size_t)d.E * 4, st, sc.ti, T, (int)d.E, k,
-                           sc.off, sc.stok, sc.pos);
-        break;
+    if (!run.perm) {
+        static_assert(kMoeChunkAssign * 4 <= 64 * 1024, "a launch's tokens fit the list in LDS");
+        static bool attr_set = false;  // idempotent attribute write; races only repeat it
+        if (!attr_set) {
+            e = (int)hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_permute_kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMoeChunkAssign * 4);
+            if (e) return e;
+            attr_set = true;
+        }
+        hipLaunchKernelGGL(moe_permute_kernel, dim3((unsigned)d.E), dim3(kMoePermThreads), (size_t)T * 4, st, sc.ti, T,
+                           (int)d.E, k, sc.off, sc.stok, sc.pos);
     }
     run.xa[0] = x_bf16 ? reinterpret_cast<const uint16_t *>(x) : sc.xb;
     run.xa[1] = x_bf16 ? nullptr : sc.xb + T * d.H;

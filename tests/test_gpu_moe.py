@@ -463,3 +463,29 @@ def test_moe_misaligned_x(O, dev):
     assert rc == 0
     torch.cuda.synchronize()
     assert torch.equal(yv, moe.forward(x, logits, top_k=k))
+
+
+# Many rows per expert: batches over 1024 tokens (permuted by one workgroup per expert, tokens past
+# a whole chunk of 1024, an expert nobody chose, every token on one expert) and batches whose
+# 64-row passes spread over several sets of workgroups (1, 2 and 4 passes' worth, a skewed load
+# with more passes than sets).
+@pytest.mark.parametrize("E,H,I,T,k,xdt,skew", [(4, 96, 64, 1025, 2, "bf16", 0), (5, 64, 96, 2500, 1, "f32", 1),
+                                               (3, 96, 96, 2048, 3, "bf16", 0), (12, 64, 64, 1100, 9, "bf16", 0),
+                                               (4, 96, 96, 65, 4, "f32", 0), (2, 64, 64, 300, 1, "bf16", 2),
+                                               (8, 96, 96, 900, 2, "bf16", 2)])
+def test_moe_many_rows_per_expert(O, dev, E, H, I, T, k, xdt, skew):
+    import nn_amd
+    L = make_layer(E, H, I, seed=E * 13 + T)
+    moe = upload(L, E, H, I)
+    x = torch.from_numpy(nn_amd.synth_normal(31, 5, (T, H), 1.0)).to(dev)
+    if xdt == "bf16":
+        x = x.to(torch.bfloat16)
+    lg = nn_amd.synth_normal(31, 6, (T, E), 1.0)
+    if skew == 1:
+        lg[:, 2] = -np.inf  # an expert without tokens
+    if skew == 2:
+        lg[:, E - 1] += 20.0  # every token on the last expert
+    y, ti, tw = moe.forward(x, torch.from_numpy(lg).to(dev), top_k=k, return_routing=True)
+    ref, rti, rtw = O.moe_forward(x.float().cpu().numpy(), lg, k, L["gp"], L["gs"], L["gb"], L["dp"], L["ds"], L["db"], I)
+    assert np.array_equal(ti.cpu().numpy().astype(np.uint32), rti), "routing differs"
+    check_close(ref, y.cpu().numpy(), f"moe many rows E={E} T={T} k={k} x={xdt} skew={skew}")
