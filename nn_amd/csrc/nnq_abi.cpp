@@ -516,11 +516,15 @@ static bool gemm_batch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
 }
 
 // the prefill GEMM's scratch for m tokens run in launches of gemm_chunk_rows rows (the
-// first launch's rows, or the last, shorter one's when that plan needs more)
-static size_t gemm_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
+// first launch's rows, or the last, shorter one's when that plan needs more).  y is the output
+// the launches get (null: any 16-byte aligned one): the wide kernels take only such outputs, and
+// the block kernel that runs in their place has other scratch.  (A later launch's y is as
+// aligned as the first's: those kernels' rows are whole 16-column tiles.)
+static size_t gemm_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype, const void *y) {
     const int64_t mc = gemm_chunk_rows(m, w->L.k), tail = m % mc;
-    size_t b = gemm_scratch_bytes(gemm_args(w, nullptr, x_dtype, mc, nullptr, nullptr, NNQ_F32));
-    if (tail) b = std::max(b, gemm_scratch_bytes(gemm_args(w, nullptr, x_dtype, tail, nullptr, nullptr, NNQ_F32)));
+    void *yp = const_cast<void *>(y);
+    size_t b = gemm_scratch_bytes(gemm_args(w, nullptr, x_dtype, mc, nullptr, yp, NNQ_F32));
+    if (tail) b = std::max(b, gemm_scratch_bytes(gemm_args(w, nullptr, x_dtype, tail, nullptr, yp, NNQ_F32)));
     return b;
 }
 
@@ -530,10 +534,10 @@ static size_t few_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype
     return gemm_few_scratch_bytes(gemm_args(w, nullptr, x_dtype, rows, nullptr, nullptr, NNQ_F32), w->L.fmt);
 }
 
-static size_t linear_scratch_bytes(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
+static size_t linear_scratch_bytes(const nnq_weight *w, int64_t m, nnq_dtype x_dtype, const void *y) {
     if (few_batch(w, m, x_dtype)) return few_call_scratch(w, m, x_dtype);
     if (!gemm_batch(w, m, x_dtype)) return 0;
-    return gemm_call_scratch(w, m, x_dtype);
+    return gemm_call_scratch(w, m, x_dtype, y);
 }
 
 // whether a prefill of m tokens can write h = silu(gate) * up from the gate | up GEMM: Q4_K, one
@@ -561,7 +565,7 @@ static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype
         Scratch s;
         void *scr = ext_scratch;
         if (!scr) {
-            HIP_TRY(s.alloc(gemm_call_scratch(w, m, x_dtype), (hipStream_t)stream), "scratch alloc");
+            HIP_TRY(s.alloc(gemm_call_scratch(w, m, x_dtype, y), (hipStream_t)stream), "scratch alloc");
             scr = s.p;
         }
         for (int64_t m0 = 0; m0 < m; m0 += mc) {
@@ -638,7 +642,7 @@ int nnq_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype, int64_t m,
     if (!array_bytes(m, k, x_dtype == NNQ_BF16 ? 2 : 4, &xbytes) ||
         !array_bytes(m, w->L.n, y_dtype == NNQ_BF16 ? 2 : 4, &ybytes))
         return size_fail();
-    const size_t lb = linear_scratch_bytes(w, m, x_dtype);
+    const size_t lb = linear_scratch_bytes(w, m, x_dtype, ym ? nullptr : y);
     const size_t sizes[3] = {xm ? xbytes : 0, ym ? ybytes : 0, lb};
     if (!plan_regions(sizes, 3, off, &total)) return size_fail();
     Scratch s;
@@ -979,9 +983,10 @@ int nnq_mlp_forward(const nnq_mlp *p, const void *x, nnq_dtype x_dtype, int64_t 
         !array_bytes(m, k, x_dtype == NNQ_BF16 ? 2 : 4, &xbytes) ||
         !array_bytes(m, p->hidden, y_dtype == NNQ_BF16 ? 2 : 4, &ybytes))
         return size_fail();
-    const size_t lin_bytes =
-        std::max(linear_scratch_bytes(p->gu, m, x_dtype), fused ? 0 : linear_scratch_bytes(p->down, m, NNQ_F32));
     const bool xm = misaligned_in(x), ym = misaligned_out(y);
+    const size_t lin_bytes =
+        std::max(linear_scratch_bytes(p->gu, m, x_dtype, nullptr),
+                 fused ? 0 : linear_scratch_bytes(p->down, m, NNQ_F32, ym ? nullptr : y));
     const size_t sizes[5] = {gu_bytes, h_bytes, lin_bytes, xm ? xbytes : 0, ym ? ybytes : 0};
     size_t off[5], total = 0;
     if (!plan_regions(sizes, 5, off, &total)) return size_fail();

@@ -200,3 +200,30 @@ def test_wide_q6k(m, n, k):
     assert err <= 1e-5, f"{m}x{n}x{k}: {err:.2e} of the row's rms"
     yb = nn_amd.quantized_linear(x, w, bias, out_dtype=torch.bfloat16)
     assert torch.equal(yb, y.to(torch.bfloat16)), "bf16 output: the f32 result rounded once"
+
+
+# An output that is 4-byte but not 16-byte aligned: the wide kernels refuse it, and the kernel that
+# runs instead has other scratch (min-term sums and more K parts' slabs), which the call has to size.
+# Bars: 2-norm error, as f32 sums give (Q4_K: offset and minimum terms cancel in them).
+@pytest.mark.parametrize("fmt,x_dtype,bar", [("q8_0", torch.bfloat16, 1e-5), ("q6_k", torch.bfloat16, 1e-5),
+                                             ("q4_k", torch.bfloat16, 5e-5), ("q4_k", torch.float32, 5e-5)])
+def test_prefill_unaligned_output(fmt, x_dtype, bar):
+    import nn_amd
+    from nn_amd import _lib
+    nn_amd.init(0)
+    m, n, k = 203, 6144, 4096
+    wf = nn_amd.synth_normal(m, 1, (n, k), 0.02)
+    b = {"q8_0": nn_amd.quantize_q8_0, "q6_k": nn_amd.quantize_q6_k, "q4_k": nn_amd.quantize_q4_k}[fmt](wf)
+    w = make_weight(fmt, b, n, k)
+    x = torch.from_numpy(nn_amd.synth_normal(m, 2, (m, k), 1.0)).cuda().to(x_dtype)
+    ref = x.double() @ w.dequantize().double().t()
+    for off in (1, 2):
+        buf = torch.full((m * n + 8,), 7.0, device="cuda")
+        y = buf[off:off + m * n]
+        assert y.data_ptr() % 16 != 0
+        rc = _lib.load().nnq_linear(w.handle, x.data_ptr(), 2 if x_dtype == torch.bfloat16 else 0, m, k, None, 0,
+                                    y.data_ptr(), 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.last_error()
+        err = ((y.double().view(m, n) - ref).norm() / ref.norm()).item()
+        assert err <= bar, f"{fmt} output at {4 * off} bytes: {err:.2e}"
+        assert (buf[:off] == 7.0).all() and (buf[off + m * n:] == 7.0).all()
