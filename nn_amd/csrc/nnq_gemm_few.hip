@@ -25,9 +25,9 @@
 // and the offset from an MFMA with a constant, 2e-7 here).  The lo product comes first: added
 // to a finished hi sum its low bits would be cut off one instruction at a time.
 // Measured (us, before -> now; before: GEMV passes or the prefill GEMM, each of which reads the
-// weight or stages the activation more than once): Q6_K LM head 151936 x 4096, 8 bf16 rows 268
-// -> 103, 16 rows 271 -> 204 (two launches); Q8_0 4096 x 4096, 12 bf16 rows 17.3 -> 7.8;
-// Q4_K 4096 x 12288, 6 f32 rows 19.0 -> 17.2 (K split three ways), 12288 x 4096, 16 f32 rows
+// weight or stages the activation more than once): Q6_K LM head 151936 x 4096, 8 bf16 rows 260
+// -> 97, 16 rows 271 -> 204 (two launches); Q8_0 4096 x 4096, 12 bf16 rows 17.3 -> 7.8;
+// Q4_K 4096 x 12288, 6 f32 rows 18.3 -> 16.0 (K split three ways), 12288 x 4096, 16 f32 rows
 // 27.3 -> 18.0.
 // Rows: Q8_0 and Q4_K have one scale per 32 k, one MFMA row per token.  A Q6_K scale covers 16 k,
 // so token t takes rows 2t and 2t + 1, each with zeros in the other sub-block's half of k.

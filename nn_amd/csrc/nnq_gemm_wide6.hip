@@ -18,8 +18,8 @@
 // other half run, a wave taking two (tile, 64-k chunk) pieces whose raw bytes were loaded half a
 // super-block earlier.  One barrier per half.  K is split over workgroups (f32 slabs summed in
 // order) when the tiles alone would leave CUs idle.
-// 512 x 4096 x 12288: 143 us in the block kernel (128 x 128 tiles, every wave decoding its own
-// columns), 111 here, 930 TFLOP/s of MFMA work.
+// 512 x 4096 x 12288 with staging and slab sum: 134 us in the block kernel (128 x 128 tiles, every
+// wave decoding its own columns), 105 here, 980 TFLOP/s of MFMA work.
 #include "nnq_device.h"
 #include "nnq_internal.h"
 
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q6k_wide_kernel(Wide6Args a) {
 // per super-block, plus the slabs; where that is not below the block kernel's estimate, that
 // kernel keeps the shape (1000 x 2048 x 2560: 57 us here, 49 there; 274 x 19200 x 7168, whose
 // second row tile is nearly all padding: 285 and 277).  Measured (block kernel -> here): 512 x
-// 4096 x 12288 143 -> 111 us, 512 x 12288 x 4096 167 -> 123, 300 x 4096 x 4096 67 -> 49, 200 x
+// 4096 x 12288 134 -> 105 us, 512 x 12288 x 4096 167 -> 123, 300 x 4096 x 4096 67 -> 49, 200 x
 // 4096 x 12288 108 -> 66, 256 x 24576 x 1024 61 -> 42.
 // Returns the K split (0: the block kernel takes the shape).
 int gemm_wide6_plan(const GemmArgs &a) {
