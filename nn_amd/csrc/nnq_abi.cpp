@@ -463,9 +463,10 @@ static int check_linear(const nnq_weight *w, const void *x, nnq_dtype xd, int64_
 }  // extern "C"
 
 // One validated linear call: the few-row GEMM (few_batch), the MFMA GEMM (gemm_batch) or GEMV
-// passes of up to 4 tokens.  GEMV-only options: x_swiglu (x holds gate | up rows of 2k f32, the input
-// is silu(gate) * up; m <= 2 so one pass) and a status (mode 1 clears it in the
-// first pass, mode 2 flags non-finite outputs in every pass).
+// passes of up to 4 tokens.  Options of a decode GEMV (m <= 2, so one pass): x_swiglu (x holds
+// gate | up rows of 2k f32, the input is silu(gate) * up) and a status (mode 1 clears it, mode 2
+// flags non-finite outputs).  They do not choose the path: a call of more tokens that gives one
+// is refused, except a swiglu_out call, whose wide GEMM clears the status.
 static GemmArgs gemm_args(const nnq_weight *w, const void *x, nnq_dtype x_dtype, int64_t m, const float *bias, void *y,
                           nnq_dtype y_dtype) {
     const Layout &L = w->L;
@@ -554,10 +555,12 @@ static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype
     if (swiglu_out && (w->L.fmt != NNQ_FMT_Q4_K || (m > 2 && !prefill_swiglu(w, m, x_dtype)) || x_swiglu || bias ||
                        w->L.n % 16))
         return fail(NNQ_ERR_INVALID_ARGUMENT, "SwiGLU epilogue needs a Q4_K decode GEMV or wide GEMM over whole tiles");
+    if (m > 2 && (x_swiglu || (status && !swiglu_out)))
+        return fail(NNQ_ERR_INVALID_ARGUMENT, "a SwiGLU input or a status needs a decode GEMV");
     const Layout &L = w->L;
     const int64_t k = L.k;
     const size_t xe = x_dtype == NNQ_BF16 ? 2 : 4, ye = y_dtype == NNQ_BF16 ? 2 : 4;
-    if (gemm_batch(w, m, x_dtype) && !x_swiglu) {
+    if (gemm_batch(w, m, x_dtype)) {
         // prefill: MFMA GEMM (Q4_K: nnq_gemm*.hip; Q8_0 / Q6_K: nnq_gemm_blk.hip), in launches
         // of gemm_chunk_rows rows (their 32-bit activation offsets; one launch up to ~43k
         // rows at K = 12288), one after another on the stream sharing the scratch
@@ -580,7 +583,7 @@ static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype
         }
         return NNQ_OK;
     }
-    if (!x_swiglu && !status && few_batch(w, m, x_dtype)) {
+    if (few_batch(w, m, x_dtype)) {
         const int64_t mc = gemm_few_rows(L.fmt);
         Scratch s;
         void *scr = ext_scratch;
@@ -943,8 +946,8 @@ static int mlp_run(const nnq_mlp *p, const void *x, nnq_dtype x_dtype, int64_t m
     const int64_t I = p->inter;
     int rc = 0;
     float *gu = reinterpret_cast<float *>(base);
-    rc = dispatch_linear(p->gu, x, x_dtype, m, nullptr, gu, NNQ_F32, stream, 0, status_dev, fused || hout ? 1 : 0, lin,
-                         hout ? 1 : 0);
+    rc = dispatch_linear(p->gu, x, x_dtype, m, nullptr, gu, NNQ_F32, stream, 0, fused || hout ? status_dev : nullptr, 1,
+                         lin, hout ? 1 : 0);
     if (rc) return rc;
     if (hout && m <= 2) return dispatch_linear(p->down, gu, NNQ_F32, m, nullptr, y, y_dtype, stream, 0, status_dev, 2);
     if (fused) return dispatch_linear(p->down, gu, NNQ_F32, m, nullptr, y, y_dtype, stream, 1, status_dev, 2);

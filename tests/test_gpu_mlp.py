@@ -130,3 +130,26 @@ def test_mlp_misaligned_x(O, dev):
         big = torch.zeros(m * H + 4, device=dev)
         big[1:1 + m * H] = x.reshape(-1)
         assert torch.equal(mlp(big[1:1 + m * H].view(m, H)), mlp(x))
+
+
+# check=True asks for the output check only: the linears are the unchecked call's at every batch size,
+# for gate | up of 96, 512 and 2048 tiles (the few-row GEMM's limits for Q4_K), so the results are
+# the same bits.
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_k", "q6_k"])
+@pytest.mark.parametrize("inter", [768, 4096, 16384])
+def test_mlp_checked_equals_unchecked(dev, fmt, inter):
+    import nn_amd
+    H = 512
+    quant = {"q8_0": nn_amd.quantize_q8_0, "q4_k": nn_amd.quantize_q4_k, "q6_k": nn_amd.quantize_q6_k}[fmt]
+    g, u, d = (quant(nn_amd.synth_normal(71, j, s, 0.03)) for j, s in ((1, (inter, H)), (2, (inter, H)),
+                                                                       (3, (H, inter))))
+    mlp = nn_amd.QuantizedMLP(g, u, d, FMT[fmt][0], H, inter, layout=FMT[fmt][1])
+    for m in (1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 16, 17, 130):
+        xf = torch.from_numpy(nn_amd.synth_normal(72 + m, 4, (m, H), 1.0)).to(dev)
+        for x in (xf, xf.to(torch.bfloat16)):
+            y = mlp(x, check=False)
+            assert torch.isfinite(y).all()
+            assert torch.equal(mlp(x), y), f"{fmt} inter={inter} m={m} x={x.dtype}"
+        xf[m - 1, 5] = float("inf")
+        with pytest.raises(nn_amd.NonFiniteData):
+            mlp(xf)
