@@ -488,27 +488,8 @@ static GemmArgs gemm_args(const nnq_weight *w, const void *x, nnq_dtype x_dtype,
     return g;
 }
 
-// The path of a linear call of m tokens, by measured crossovers on MI355X (us, x f32 / bf16):
-//  - 1 and 2 tokens: one decode-GEMV pass;
-//  - 3 to 16: the few-row GEMM (few_batch), which reads the weight once, from 5 tokens on
-//    (Q8_0 4096x4096, 12 tokens: 14.3 / 17.0 as passes / GEMM, 12.8 / 7.5 here; Q6_K
-//    12288x4096, 8 tokens: 26.8 / 26.3 as two passes, 14.0 / 12.1).  Below that a GEMV pass of
-//    4 tokens has the shorter prologue (Q6_K 4096x4096: 6.2 against 8.4 / 7.4), except over
-//    many tiles per CU (4 tokens, Q6_K: 24576 rows 23.8 against 20.3, 60000 rows 56 against 42;
-//    Q8_0: 24576 rows level, 60000 rows 46.6 against 43.4).  Q4_K with f32 x takes it from 7
-//    tokens (4096x4096: 5 and 6 as two passes 8.6 and 9.0 against 9.1 and 9.3; 8: 10.5 against
-//    9.6), from 5 with two tiles per CU (24576 rows: 30.0 against 19.3) or K over 8192 (6
-//    tokens at 4096x12288: 19.0 against 17.2).  Q4_K with bf16 x keeps the thin GEMM, which
-//    stages nothing, up to that many tiles (16 tokens: 12288x4096 10.0 against 13.0, 24576
-//    rows 18.8 against 19.5, 60000 rows 45.2 against 37.6);
-//  - other counts: the MFMA GEMM.
 static bool few_batch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
-    const Layout &L = w->L;
-    if (m < 3 || m > 16 || L.k > ((int64_t)1 << 24) || L.ntile >= ((int64_t)1 << 31)) return false;
-    if (L.ntile >= 2048) return true;  // eight tiles per CU
-    if (L.fmt != NNQ_FMT_Q4_K) return m > 4;
-    if (x_dtype == NNQ_BF16) return false;
-    return m > 6 || (m > 4 && (L.ntile >= 512 || L.k > 8192));
+    return nnq_rule_few_rows(w->L.fmt, w->L.ntile, w->L.k, m, x_dtype == NNQ_BF16) != 0;
 }
 
 static bool gemm_batch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {

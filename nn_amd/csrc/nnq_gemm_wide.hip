@@ -690,44 +690,12 @@ __global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const void *xv, in
 
 }  // namespace
 
-// The wide kernel's shape rules: more than 128 rows (below, half of a 256-row tile or more is
-// padding: f32 x, 100 x 4096 x 12288 109 us against the ring's 51), whole 16-row weight tiles
-// and a 16-byte aligned output (the epilogue writes 16-byte row chunks), K <= 4096 * 3 (the
-// staging keeps the row in one workgroup's registers and its sub-block sums in LDS), and at
-// least 128 workgroups.  Column tiles per workgroup (6, 4 or 8) and K split (1 to 8 equal parts
-// of whole super-blocks) are the ones with the least estimated time: rounds of workgroups over
-// the CUs, each 3 us and its super-blocks times the measured time of one (us, 6, 4 and 8 tiles: bf16 x
-// 3.8, 3.0 and 5.0, f32 x 6.2, 5.2 and 7.8: more tiles read each A fragment less often), plus
-// the slabs' write, read and launch.  512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles;
-// the ring kernel over two planes 153) and 115 at 4096 x 12288 (8 tiles, K in four; 4 tiles
-// and K in two 134, ring 155), of bf16 x there 77 (4 tiles 83); 203 rows of f32 x at 12288 x
-// 4096 take 6 tiles and K in two (256 workgroups).
-// With random x these rates are the chip's power limit for f16 products: a library f16 GEMM
-// of 512 x 12288 x 4096 takes 58 us (44 with x = 0), this kernel 66 with its staging (60).
-// Returns the column tiles per workgroup (0: the ring kernel takes the shape) and the K split.
+// The wide kernel's column tiles per workgroup (0: the ring kernel takes the call) and K split:
+// the rule of its shape (nnq_rule_gemm_wide), for whole 16-row weight tiles and a 16-byte aligned
+// output (the epilogue writes 16-byte row chunks).
 int gemm_wide_plan(const GemmArgs &a, int *ks) {
-    if (a.blk || a.m <= 128 || a.k > 4096 * 3 || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
-    const int64_t nrt = (a.m + BM - 1) / BM;
-    const float sb_us[2][3] = {{3.8f, 3.0f, 5.0f}, {6.2f, 5.2f, 7.8f}};
-    float best = 0.0f;
-    int nt = 0;
-    for (int i = 0; i < 3; i++) {
-        const int c = i == 0 ? 6 : i == 1 ? 4 : 8;
-        if (a.ntile % c) continue;
-        for (int split = 1; split <= 8; split++) {
-            const int64_t wg = nrt * (a.ntile / c) * split;
-            if (wg < 128 || a.nblk % split || a.nblk / split < 2) continue;
-            const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(a.m * a.n) * 4.0f / 4.0e6f : 0.0f;
-            const float us =
-                (float)((wg + 255) / 256) * (3.0f + (float)(a.nblk / split) * sb_us[a.x_bf16 ? 0 : 1][i]) + slabs;
-            if (!nt || us < best) {
-                best = us;
-                nt = c;
-                if (ks) *ks = split;
-            }
-        }
-    }
-    return nt;
+    if (a.blk || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
+    return nnq_rule_gemm_wide(a.m, a.ntile, a.nblk, a.x_bf16, ks);
 }
 
 // whether the call can write silu(gate) * up (swiglu_out) from the wide kernel's epilogue

@@ -244,35 +244,11 @@ __global__ __launch_bounds__(NTH, 1) void gemm_q6k_wide_kernel(Wide6Args a) {
 
 }  // namespace
 
-// Shape rules: Q6_K, bf16 activations, more than 128 rows, whole groups of 8 weight tiles, K up
-// to 4096 * 3 (the activation staging), a 16-byte aligned output, and at least 192 workgroups, or
-// 128 with 8 super-blocks each.  The K split (1 to 8 equal parts of two or more super-blocks) is
-// the one with the least estimated time: rounds of workgroups over the CUs, each 3 us and 7.8 us
-// per super-block, plus the slabs; where that is not below the block kernel's estimate, that
-// kernel keeps the shape (1000 x 2048 x 2560: 57 us here, 49 there; 274 x 19200 x 7168, whose
-// second row tile is nearly all padding: 285 and 277).  Measured (block kernel -> here): 512 x
-// 4096 x 12288 134 -> 105 us, 512 x 12288 x 4096 167 -> 123, 300 x 4096 x 4096 67 -> 49, 200 x
-// 4096 x 12288 108 -> 66, 256 x 24576 x 1024 61 -> 42.
-// Returns the K split (0: the block kernel takes the shape).
+// The K split (0: the block kernel takes the call): the rule of its shape (nnq_rule_gemm_wide6), for
+// Q6_K, bf16 activations, whole 16-row weight tiles and a 16-byte aligned output.
 int gemm_wide6_plan(const GemmArgs &a) {
-    if (a.blk != NNQ_FMT_Q6_K || !a.x_bf16 || a.m <= 128 || a.k > 4096 * 3 || a.ntile % TL || a.n != a.ntile * 16 ||
-        (reinterpret_cast<uintptr_t>(a.y) & 15))
-        return 0;
-    const int64_t base = (a.m + BM - 1) / BM * (a.ntile / TL);
-    // the block kernel: 128-row tiles at about 350 TFLOP/s, its staging and slab sum 12 us
-    float best = 12.0f + 2.0f * (float)((a.m + 127) / 128 * 128) * (float)a.n * (float)a.k / 350.0e6f;
-    int ks = 0;
-    for (int split = 1; split <= 8; split++) {
-        const int64_t wg = base * split;
-        if (a.nblk % split || wg < 128 || a.nblk / split < 2 || (wg < 192 && a.nblk / split < 8)) continue;
-        const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(a.m * a.n) * 4.0f / 4.0e6f : 0.0f;
-        const float us = (float)((wg + 255) / 256) * (3.0f + (float)(a.nblk / split) * 7.8f) + slabs;
-        if (us < best) {
-            best = us;
-            ks = split;
-        }
-    }
-    return ks;
+    if (a.blk != NNQ_FMT_Q6_K || !a.x_bf16 || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
+    return nnq_rule_gemm_wide6(a.m, a.ntile, a.nblk);
 }
 
 // scratch: the staged activation | rowback | slabs

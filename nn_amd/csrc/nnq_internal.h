@@ -74,6 +74,17 @@ int64_t moe_chunk_tokens(int64_t tokens, int top_k);
 // 4 * rows * k < 2^31
 int64_t gemm_chunk_rows(int64_t m, int64_t k);
 
+// Rules that choose a kernel by sizes alone (nnq_plan.cpp), with C names so that a test can ask
+// which kernel a shape takes.  ntile: 16-row weight tiles, nblk: super-blocks of 256 along K.
+constexpr int kMoeFewT = 16;        // moe_few_kernel: most tokens
+constexpr int kMoeFewAssign = 128;  //   and assignments (two per lane of its ballots)
+extern "C" {
+int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16);  // 1: gemm_few_kernel
+int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *ks);
+int nnq_rule_gemm_wide6(int64_t m, int64_t ntile, int64_t nblk);
+int nnq_rule_moe_few(int64_t experts, int64_t hidden, int64_t inter, int64_t tokens, int top_k, int x_bf16);
+}
+
 // ---- kernel launch parameters ------------------------------------------------------
 struct GemvArgs {
     const uint8_t *qs;    // quant plane

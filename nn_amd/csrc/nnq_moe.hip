@@ -1010,8 +1010,6 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
 // 47 us of which its loads alone 24: the rest is the conversion (24 VALU per k-block and
 // column block) and the barrier per item.  One-shot workgroups without the loop: 136 us.
 // ---------------------------------------------------------------------------------
-constexpr int kMoeFewT = 16;        // tokens
-constexpr int kMoeFewAssign = 128;  // assignments: two per lane of the ballots
 constexpr int kMoeFewWaves = 8;
 constexpr int kMoeFewRows = 4;    // rows of an item
 constexpr int kMoeFewKb = 6;      // most k-blocks of a batch
@@ -1525,7 +1523,7 @@ int launch_moe(const MoeDev &d, const void *x, int x_bf16, int64_t T, const floa
     run.T = T;
     run.k = k;
     run.perm = T <= kMoeInPermT ? 1 : 0;
-    const bool few = T <= kMoeFewT && run.A <= kMoeFewAssign;
+    const bool few = nnq_rule_moe_few(d.E, d.H, d.I, T, k, x_bf16) != 0;
     if (d.E <= 256)
         hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, logits, nsplit, bias, T,
                            (int)d.E, k, sc.ti, sc.tw, topk_idx, topk_w);

@@ -1,5 +1,6 @@
 // Host arithmetic of the C ABI's calls: the byte sizes of token arrays, the layout of a
-// call's workspace regions, and how long batches are cut into launches.  It is kept apart
+// call's workspace regions, how long batches are cut into launches, and the rules that choose
+// a kernel by sizes alone.  It is kept apart
 // from nnq_abi.cpp (which makes the HIP runtime calls) so that the sanitizer harness
 // (tests/sanitize) runs the same code on the CPU over ragged and extreme shapes.
 #include <algorithm>
@@ -45,6 +46,105 @@ int64_t gemm_chunk_rows(int64_t m, int64_t k) {
     int64_t rows = lim / (4 * k);
     if (rows >= 256) rows = rows / 256 * 256;  // whole 256-row tiles per launch
     return std::min(m, std::max<int64_t>(1, rows));
+}
+
+// ---- dispatch rules ----------------------------------------------------------------
+
+// The path of a linear call of m tokens, by measured crossovers on MI355X (us, x f32 / bf16):
+//  - 1 and 2 tokens: one decode-GEMV pass;
+//  - 3 to 16: the few-row GEMM (nnq_gemm_few.hip) from 5 tokens on (Q8_0 4096x4096, 12 tokens:
+//    14.3 / 17.0 as passes / GEMM, 12.8 / 7.5 there; Q6_K 12288x4096, 8 tokens: 26.8 / 26.3 as
+//    two passes, 14.0 / 12.1).  Below that a GEMV pass of
+//    4 tokens has the shorter prologue (Q6_K 4096x4096: 6.2 against 8.4 / 7.4), except over
+//    many tiles per CU (4 tokens, Q6_K: 24576 rows 23.8 against 20.3, 60000 rows 56 against 42;
+//    Q8_0: 24576 rows level, 60000 rows 46.6 against 43.4).  Q4_K with f32 x takes it from 7
+//    tokens (4096x4096: 5 and 6 as two passes 8.6 and 9.0 against 9.1 and 9.3; 8: 10.5 against
+//    9.6), from 5 with two tiles per CU (24576 rows: 30.0 against 19.3) or K over 8192 (6
+//    tokens at 4096x12288: 19.0 against 17.2).  Q4_K with bf16 x keeps the thin GEMM, which
+//    stages nothing, up to that many tiles (16 tokens: 12288x4096 10.0 against 13.0, 24576
+//    rows 18.8 against 19.5, 60000 rows 45.2 against 37.6);
+//  - other counts: the MFMA GEMM.
+// 1 where the few-row GEMM takes the call.
+int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16) {
+    if (m < 3 || m > 16 || k > ((int64_t)1 << 24) || ntile >= ((int64_t)1 << 31)) return 0;
+    if (ntile >= 2048) return 1;  // eight tiles per CU
+    if (fmt != NNQ_FMT_Q4_K) return m > 4;
+    if (x_bf16) return 0;
+    return m > 6 || (m > 4 && (ntile >= 512 || k > 8192));
+}
+
+// The wide kernel's shape rules: more than 128 rows (below, half of a 256-row tile or more is
+// padding: f32 x, 100 x 4096 x 12288 109 us against the ring's 51), whole 16-row weight tiles
+// and a 16-byte aligned output (the epilogue writes 16-byte row chunks), K <= 4096 * 3 (the
+// staging keeps the row in one workgroup's registers and its sub-block sums in LDS), and at
+// least 128 workgroups.  Column tiles per workgroup (6, 4 or 8) and K split (1 to 8 equal parts
+// of whole super-blocks) are the ones with the least estimated time: rounds of workgroups over
+// the CUs, each 3 us and its super-blocks times the measured time of one (us, 6, 4 and 8 tiles: bf16 x
+// 3.8, 3.0 and 5.0, f32 x 6.2, 5.2 and 7.8: more tiles read each A fragment less often), plus
+// the slabs' write, read and launch.  512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles;
+// the ring kernel over two planes 153) and 115 at 4096 x 12288 (8 tiles, K in four; 4 tiles
+// and K in two 134, ring 155), of bf16 x there 77 (4 tiles 83); 203 rows of f32 x at 12288 x
+// 4096 take 6 tiles and K in two (256 workgroups).
+// With random x these rates are the chip's power limit for f16 products: a library f16 GEMM
+// of 512 x 12288 x 4096 takes 58 us (44 with x = 0), this kernel 66 with its staging (60).
+// Returns the column tiles per workgroup (0: the ring kernel takes the shape) and the K split.
+int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *ks) {
+    if (m <= 128 || nblk > 48) return 0;
+    const int64_t nrt = (m + 255) / 256, n = ntile * 16;
+    const float sb_us[2][3] = {{3.8f, 3.0f, 5.0f}, {6.2f, 5.2f, 7.8f}};
+    float best = 0.0f;
+    int nt = 0;
+    for (int i = 0; i < 3; i++) {
+        const int c = i == 0 ? 6 : i == 1 ? 4 : 8;
+        if (ntile % c) continue;
+        for (int split = 1; split <= 8; split++) {
+            const int64_t wg = nrt * (ntile / c) * split;
+            if (wg < 128 || nblk % split || nblk / split < 2) continue;
+            const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(m * n) * 4.0f / 4.0e6f : 0.0f;
+            const float us = (float)((wg + 255) / 256) * (3.0f + (float)(nblk / split) * sb_us[x_bf16 ? 0 : 1][i]) + slabs;
+            if (!nt || us < best) {
+                best = us;
+                nt = c;
+                if (ks) *ks = split;
+            }
+        }
+    }
+    return nt;
+}
+
+// The wide Q6_K kernel's shape rules: bf16 activations, more than 128 rows, whole groups of 8 weight tiles, K up
+// to 4096 * 3 (the activation staging), a 16-byte aligned output, and at least 192 workgroups, or
+// 128 with 8 super-blocks each.  The K split (1 to 8 equal parts of two or more super-blocks) is
+// the one with the least estimated time: rounds of workgroups over the CUs, each 3 us and 7.8 us
+// per super-block, plus the slabs; where that is not below the block kernel's estimate, that
+// kernel keeps the shape (1000 x 2048 x 2560: 57 us wide, 49 there; 274 x 19200 x 7168, whose
+// second row tile is nearly all padding: 285 and 277).  Measured (block kernel -> wide): 512 x
+// 4096 x 12288 134 -> 105 us, 512 x 12288 x 4096 167 -> 123, 300 x 4096 x 4096 67 -> 49, 200 x
+// 4096 x 12288 108 -> 66, 256 x 24576 x 1024 61 -> 42.
+// Returns the K split (0: the block kernel takes the shape).
+int nnq_rule_gemm_wide6(int64_t m, int64_t ntile, int64_t nblk) {
+    if (m <= 128 || nblk > 48 || ntile % 8) return 0;
+    const int64_t base = (m + 255) / 256 * (ntile / 8), n = ntile * 16;
+    // the block kernel: 128-row tiles at about 350 TFLOP/s, its staging and slab sum 12 us
+    float best = 12.0f + 2.0f * (float)((m + 127) / 128 * 128) * (float)n * (float)(nblk * 256) / 350.0e6f;
+    int ks = 0;
+    for (int split = 1; split <= 8; split++) {
+        const int64_t wg = base * split;
+        if (nblk % split || wg < 128 || nblk / split < 2 || (wg < 192 && nblk / split < 8)) continue;
+        const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(m * n) * 4.0f / 4.0e6f : 0.0f;
+        const float us = (float)((wg + 255) / 256) * (3.0f + (float)(nblk / split) * 7.8f) + slabs;
+        if (us < best) {
+            best = us;
+            ks = split;
+        }
+    }
+    return ks;
+}
+
+// Whether a MoE layer's experts run as moe_few_kernel's items: up to kMoeFewT tokens and
+// kMoeFewAssign assignments.
+int nnq_rule_moe_few(int64_t experts, int64_t hidden, int64_t inter, int64_t tokens, int top_k, int x_bf16) {
+    return tokens <= kMoeFewT && tokens * top_k <= kMoeFewAssign;
 }
 
 }  // namespace nnq

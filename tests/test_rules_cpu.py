@@ -1,0 +1,61 @@
+"""The rules that choose a kernel by sizes alone (nn_amd/csrc/nnq_plan.cpp), asked through their C names:
+what holds for every shape.  No GPU needed."""
+import ctypes
+import random
+
+import pytest
+
+Q8_0, Q4_K, Q6_K = 8, 12, 14
+i64, c_int = ctypes.c_int64, ctypes.c_int
+
+
+@pytest.fixture(scope="module")
+def rules():
+    from nn_amd import _lib
+    lib = _lib.load()
+    lib.nnq_rule_few_rows.argtypes = [c_int, i64, i64, i64, c_int]
+    lib.nnq_rule_gemm_wide.argtypes = [i64, i64, i64, c_int, ctypes.POINTER(c_int)]
+    lib.nnq_rule_gemm_wide6.argtypes = [i64, i64, i64]
+    lib.nnq_rule_moe_few.argtypes = [i64, i64, i64, i64, c_int, c_int]
+
+    class Rules:
+        @staticmethod
+        def few_rows(fmt, m, n, k, bf16):
+            return lib.nnq_rule_few_rows(fmt, (n + 15) // 16, k, m, bf16)
+
+        @staticmethod
+        def wide(m, n, k, bf16):
+            """(column tiles per workgroup, K split); (0, 0) where the wide Q4_K kernel does not take it"""
+            ks = c_int(0)
+            return lib.nnq_rule_gemm_wide(m, n // 16, k // 256, bf16, ctypes.byref(ks)), ks.value
+
+        @staticmethod
+        def wide6(m, n, k):
+            return lib.nnq_rule_gemm_wide6(m, n // 16, k // 256)
+
+        @staticmethod
+        def moe_few(experts, hidden, inter, tokens, top_k, bf16):
+            return lib.nnq_rule_moe_few(experts, hidden, inter, tokens, top_k, bf16)
+
+    return Rules
+
+
+def test_kernel_limits(rules):
+    """No rule sends a kernel what it cannot run: rows of the few-row GEMM, tiles and K parts that divide
+    the weight, two super-blocks a part, the staging's K, the few-token kernel's ballots and rows."""
+    rng = random.Random(3)
+    for _ in range(20000):
+        m, tiles, nblk, bf16 = rng.randint(1, 3000), rng.randint(1, 4096), rng.randint(1, 64), rng.randint(0, 1)
+        n, k = 16 * tiles, 256 * nblk
+        nt, ks = rules.wide(m, n, k, bf16)
+        if nt:
+            assert m > 128 and k <= 12288 and nt in (4, 6, 8) and tiles % nt == 0 and nblk % ks == 0 and nblk // ks >= 2
+        ks = rules.wide6(m, n, k)
+        if ks:
+            assert m > 128 and k <= 12288 and tiles % 8 == 0 and nblk % ks == 0 and nblk // ks >= 2
+        for fmt in (Q8_0, Q4_K, Q6_K):
+            if rules.few_rows(fmt, m, n, k, bf16):
+                assert 3 <= m <= 16
+        experts, top_k, tokens = rng.randint(1, 300), rng.randint(1, 16), rng.randint(1, 40)
+        if top_k <= experts and rules.moe_few(experts, 32 * rng.randint(1, 200), 32 * rng.randint(1, 200), tokens, top_k, bf16):
+            assert tokens <= 16 and tokens * top_k <= 128
