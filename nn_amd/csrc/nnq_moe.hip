@@ -11,7 +11,7 @@
 //   gate_up  grouped GEMM over experts: x rows of the expert x W_gu[e] (+ bias), with
 //            the SwiGLU epilogue clamp(silu(gate), -limit, limit) * up fused in
 //   down     grouped GEMM over experts: h x W_down[e] (+ bias)
-//            (gate_up and down of up to 16 tokens: moe_few_kernel, else moe_stream_kernel)
+//            (gate_up and down of a few tokens, nnq_rule_moe_few: moe_few_kernel, else moe_stream_kernel)
 //   combine  y[t] = sum of w * y_e[t] over the token's experts in ascending expert
 //            order, the order of moe_forward's index_add (:171-189)
 //
@@ -1004,9 +1004,9 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
 // no permutation: a workgroup finds its experts in order of first appearance among the
 // assignments, by ballots over the routed experts.
 // The GPT-OSS layer (32 experts, top 4, 2880 x 2880) with its router: 1 token 107 -> 32 us,
-// 4 tokens 116 -> 59, 8 tokens 121 -> 91, 16 tokens 124 -> 112 (64 experts of 2880 x 1440,
-// top 8, 16 tokens: 163 -> 129); at 16 tokens most experts are in use and the two
-// organisations meet, so the rule (few, launch_moe) stops there.  At 8 tokens gate_up takes
+// 4 tokens 116 -> 59, 8 tokens 121 -> 91.  An expert of more than four rows is streamed and
+// converted again for each four of them, so the time grows with the rows while moe_stream_kernel's
+// does not; where the two cross is the rule nnq_rule_moe_few.  At 8 tokens gate_up takes
 // 47 us of which its loads alone 24: the rest is the conversion (24 VALU per k-block and
 // column block) and the barrier per item.  One-shot workgroups without the loop: 136 us.
 // ---------------------------------------------------------------------------------

@@ -4,6 +4,7 @@
 // from nnq_abi.cpp (which makes the HIP runtime calls) so that the sanitizer harness
 // (tests/sanitize) runs the same code on the CPU over ragged and extreme shapes.
 #include <algorithm>
+#include <cmath>
 
 #include "nnq_internal.h"
 
@@ -141,10 +142,35 @@ int nnq_rule_gemm_wide6(int64_t m, int64_t ntile, int64_t nblk) {
     return ks;
 }
 
-// Whether a MoE layer's experts run as moe_few_kernel's items: up to kMoeFewT tokens and
-// kMoeFewAssign assignments.
+// Whether a MoE layer's experts run as moe_few_kernel's items (up to kMoeFewT tokens and
+// kMoeFewAssign assignments) rather than as moe_stream_kernel's workgroups.  The items' time grows
+// with the passes of four rows over an expert's weights, expected here for even routing; the
+// streams' hardly does (a pass of theirs is 64 rows), so there is a number of passes where they
+// cross: 28 with bf16 x and 22.5 with f32 x (which the items split on each pass, the streams
+// once) for 2880 x 2880 experts, 5 and 4.5 more with each halving of an expert (an item of a small
+// one is mostly its fixed part).  Streams of over 32 experts are more workgroups than CUs, and over
+// 96 column streams take a wave more than one each: both raise it.  Measured (us, streams / items,
+// top 8): 32 experts of 2880 x 2880, 6 bf16 tokens 104 / 99, 12 108 / 123, 16 109 / 151, 4 f32 tokens
+// 127 / 127, 16 132 / 238; 16 such experts, 10 bf16 tokens 100 / 96, 16 101 / 126; 32 of 2048 x 2048, 12
+// bf16 tokens 94 / 90, 16 94 / 109; 64 of 1024 x 768, 16 f32 tokens 79 / 71.
 int nnq_rule_moe_few(int64_t experts, int64_t hidden, int64_t inter, int64_t tokens, int top_k, int x_bf16) {
-    return tokens <= kMoeFewT && tokens * top_k <= kMoeFewAssign;
+    if (tokens > kMoeFewT || tokens * top_k > kMoeFewAssign) return 0;
+    // an expert's rows are binomial: P(n) from P(n - 1)
+    const double p = (double)top_k / (double)experts;
+    double passes = (double)((tokens + 3) / 4);
+    if (p < 1.0) {
+        double pn = std::pow(1.0 - p, (double)tokens);
+        passes = 0.0;
+        for (int64_t n = 1; n <= tokens; n++) {
+            pn *= (double)(tokens - n + 1) / (double)n * p / (1.0 - p);
+            passes += pn * (double)((n + 3) / 4);
+        }
+    }
+    passes *= (double)experts;
+    const double halvings = std::max(0.0, std::log2(2880.0 * 2880.0 / ((double)hidden * (double)inter)));
+    const double cross = x_bf16 ? 28.0 + 5.0 * halvings : 22.5 + 4.5 * halvings;
+    const int64_t sets = (experts + 31) / 32, rounds = (inter / 32 + 95) / 96 + (hidden / 32 + 95) / 96;
+    return passes <= cross * (1.0 + 1.25 * (double)(sets - 1)) * 0.5 * (double)rounds;
 }
 
 }  // namespace nnq

@@ -59,3 +59,36 @@ def test_kernel_limits(rules):
         experts, top_k, tokens = rng.randint(1, 300), rng.randint(1, 16), rng.randint(1, 40)
         if top_k <= experts and rules.moe_few(experts, 32 * rng.randint(1, 200), 32 * rng.randint(1, 200), tokens, top_k, bf16):
             assert tokens <= 16 and tokens * top_k <= 128
+
+
+# Layers measured on both kernels, those of 1.1x or more between them (us, moe_stream_kernel / moe_few_kernel).
+@pytest.mark.parametrize("experts,hidden,inter,tokens,top_k,bf16,few", [
+    (32, 2880, 2880, 1, 4, 1, 1),    # 93 / 27
+    (32, 2880, 2880, 8, 4, 1, 1),    # 99 / 81
+    (32, 2880, 2880, 12, 8, 1, 0),   # 108 / 123
+    (32, 2880, 2880, 16, 8, 1, 0),   # 109 / 151
+    (32, 2880, 2880, 16, 4, 0, 0),   # 127 / 161
+    (32, 2880, 2880, 16, 8, 0, 0),   # 132 / 238
+    (16, 2880, 2880, 16, 4, 1, 1),   # 98 / 80
+    (16, 2880, 2880, 16, 8, 1, 0),   # 101 / 126
+    (16, 2880, 2880, 16, 8, 0, 0),   # 126 / 201
+    (8, 2880, 2880, 12, 8, 1, 1),    # 103 / 81
+    (8, 2880, 2880, 16, 8, 0, 0),    # 125 / 164
+    (32, 2048, 2048, 8, 4, 1, 1),    # 92 / 61
+    (32, 2048, 2048, 16, 8, 0, 0),   # 99 / 150
+    (32, 768, 2880, 16, 8, 0, 0),    # 67 / 91
+    (48, 2048, 1408, 16, 6, 0, 1),   # 156 / 110
+    (64, 2880, 1440, 16, 8, 0, 1),   # 185 / 161
+    (8, 4096, 14336, 16, 2, 0, 1),   # 985 / 352
+])
+def test_moe_few_where_it_is_faster(rules, experts, hidden, inter, tokens, top_k, bf16, few):
+    assert rules.moe_few(experts, hidden, inter, tokens, top_k, bf16) == few
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("experts,hidden,inter,top_k", [(1, 32, 32, 1), (8, 2880, 2880, 8), (32, 2880, 2880, 4),
+                                                        (4096, 32768, 32768, 8)])
+def test_moe_few_is_a_limit_in_tokens(rules, experts, hidden, inter, top_k, bf16):
+    """More tokens never bring the few-token kernel back, and one token always takes it."""
+    got = [rules.moe_few(experts, hidden, inter, t, top_k, bf16) for t in range(1, 20)]
+    assert got[0] == 1 and got == sorted(got, reverse=True) and not any(got[16:])
