@@ -55,19 +55,25 @@ int64_t gemm_chunk_rows(int64_t m, int64_t k) {
 //  - 1 and 2 tokens: one decode-GEMV pass;
 //  - 3 to 16: the few-row GEMM (nnq_gemm_few.hip) from 5 tokens on (Q8_0 4096x4096, 12 tokens:
 //    14.3 / 17.0 as passes / GEMM, 12.8 / 7.5 there; Q6_K 12288x4096, 8 tokens: 26.8 / 26.3 as
-//    two passes, 14.0 / 12.1).  Below that a GEMV pass of
-//    4 tokens has the shorter prologue (Q6_K 4096x4096: 6.2 against 8.4 / 7.4), except over
-//    many tiles per CU (4 tokens, Q6_K: 24576 rows 23.8 against 20.3, 60000 rows 56 against 42;
-//    Q8_0: 24576 rows level, 60000 rows 46.6 against 43.4).  Q4_K with f32 x takes it from 7
+//    two passes, 14.0 / 12.1).  Below that a GEMV pass of 4 tokens has the shorter prologue
+//    (Q6_K 4096x4096: 6.2 against 8.4 / 7.4), except over eight tiles per CU or more (3 f32 tokens,
+//    pass against few rows: Q6_K 151936 x 4096 133 / 97, 40960 x 2048 19.9 / 17.6; Q8_0 40960 x 2048
+//    19.0 / 16.8; Q4_K 40960 x 4096 29.2 / 24.5; under 2048 k the pass is faster, 40960 x 1024
+//    11.3 / 12.1, 10.8 / 11.3 and 8.7 / 11.4, but its sums are the less exact ones, so that the
+//    rule has no line there).  Q4_K with f32 x takes it from 7
 //    tokens (4096x4096: 5 and 6 as two passes 8.6 and 9.0 against 9.1 and 9.3; 8: 10.5 against
 //    9.6), from 5 with two tiles per CU (24576 rows: 30.0 against 19.3) or K over 8192 (6
 //    tokens at 4096x12288: 19.0 against 17.2).  Q4_K with bf16 x keeps the thin GEMM, which
 //    stages nothing, up to that many tiles (16 tokens: 12288x4096 10.0 against 13.0, 24576
-//    rows 18.8 against 19.5, 60000 rows 45.2 against 37.6);
+//    rows 18.8 against 19.5, 60000 rows 45.2 against 37.6).  Over 8 tokens of Q6_K are two
+//    launches there: four tiles per CU of one or two units leave them to the MFMA GEMM (16 bf16
+//    tokens, GEMM against few rows: 65536 x 256 14.4 / 25.4, x 512 20.7 / 26.5, x 1024 33.9 / 29.4;
+//    8192 x 512 13.7 / 11.3);
 //  - other counts: the MFMA GEMM.
 // 1 where the few-row GEMM takes the call.
 int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16) {
     if (m < 3 || m > 16 || k > ((int64_t)1 << 24) || ntile >= ((int64_t)1 << 31)) return 0;
+    if (fmt == NNQ_FMT_Q6_K && m > 8 && ntile >= 1024 && k <= 512) return 0;
     if (ntile >= 2048) return 1;  // eight tiles per CU
     if (fmt != NNQ_FMT_Q4_K) return m > 4;
     if (x_bf16) return 0;

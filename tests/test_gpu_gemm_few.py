@@ -50,6 +50,18 @@ def test_few_rows(m, n, k, fmt, xdt):
     assert torch.equal(yb, y.to(torch.bfloat16)), "bf16 output is the f32 result rounded once"
 
 
+# More than 8 rows of Q6_K are two launches: four tiles per CU of one or two units take the MFMA GEMM
+# instead (one tile below the limit, at it, and past it with a ragged last tile).
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(9, 16368, 512), (9, 16369, 512), (16, 16400, 256), (12, 16384, 768)])
+def test_q6_k_two_launches_or_gemm(m, n, k, xdt):
+    import nn_amd
+    nn_amd.init(0)
+    qw = weight("q6_k", n, k, 45)
+    x = torch.from_numpy(nn_amd.synth_normal(47, m, (m, k), 1.0)).cuda().to(xdt)
+    check(nn_amd.quantized_linear(x, qw), x.double() @ qw.dequantize().double().t(), f"q6_k {m}x{n}x{k} {xdt}")
+
+
 @pytest.mark.parametrize("m,n,k", [(5, 300, 96), (16, 40, 4128), (8, 64, 4096 + 32), (13, 48, 8192 + 224)])
 def test_few_rows_q8_0_partial_unit(m, n, k):
     import nn_amd

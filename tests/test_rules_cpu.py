@@ -92,3 +92,24 @@ def test_moe_few_is_a_limit_in_tokens(rules, experts, hidden, inter, top_k, bf16
     """More tokens never bring the few-token kernel back, and one token always takes it."""
     got = [rules.moe_few(experts, hidden, inter, t, top_k, bf16) for t in range(1, 20)]
     assert got[0] == 1 and got == sorted(got, reverse=True) and not any(got[16:])
+
+
+# Linears measured both ways, most with 1.1x or more between them (us, GEMV passes or MFMA GEMM / few-row GEMM).
+@pytest.mark.parametrize("fmt,m,n,k,bf16,few", [
+    (Q4_K, 3, 151936, 1024, 0, 1),   # 28.4 / 25.4
+    (Q4_K, 4, 32768, 3072, 0, 1),    # 18.9 / 17.0
+    (Q4_K, 3, 40960, 256, 1, 1),     # 13.3 / 10.1 (thin GEMM)
+    (Q6_K, 3, 65536, 2048, 1, 1),    # 29.6 / 23.8
+    (Q8_0, 3, 151936, 1024, 0, 1),   # 34.7 / 29.7
+    (Q6_K, 16, 65536, 256, 0, 0),    # 18.7 / 27.1
+    (Q6_K, 16, 32768, 512, 1, 0),    # 13.8 / 18.4
+    (Q6_K, 16, 65536, 1024, 0, 1),   # 46.2 / 33.2
+    (Q6_K, 16, 8192, 512, 1, 1),     # 13.7 / 11.3
+    (Q6_K, 8, 65536, 256, 1, 1),
+    (Q8_0, 16, 65536, 256, 1, 1),
+    (Q4_K, 6, 4096, 4096, 0, 0),
+    (Q4_K, 6, 4096, 12288, 0, 1),    # 19.0 / 17.2
+    (Q4_K, 16, 12288, 4096, 1, 0),   # 10.0 / 13.0 (thin GEMM)
+])
+def test_few_rows_where_they_are_faster(rules, fmt, m, n, k, bf16, few):
+    assert rules.few_rows(fmt, m, n, k, bf16) == few
