@@ -125,7 +125,9 @@ int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *
 // the one with the least estimated time: rounds of workgroups over the CUs, each 3 us and 7.8 us
 // per super-block, plus the slabs; where that is not below the block kernel's estimate, that
 // kernel keeps the shape (1000 x 2048 x 2560: 57 us wide, 49 there; 274 x 19200 x 7168, whose
-// second row tile is nearly all padding: 285 and 277).  Measured (block kernel -> wide): 512 x
+// second row tile is nearly all padding: 285 and 277).  A second 128-row tile of up to 32 rows
+// costs the block kernel less than a full one, 12% in its estimate (256, 160 and 129 x 40960 x
+// 1024: 88, 62 and 59 us, wide 69, 67 and 66; 129 x 9728 x 2560: 45.7, wide 47.9).  Measured (block kernel -> wide): 512 x
 // 4096 x 12288 134 -> 105 us, 512 x 12288 x 4096 167 -> 123, 300 x 4096 x 4096 67 -> 49, 200 x
 // 4096 x 12288 108 -> 66, 256 x 24576 x 1024 61 -> 42.
 // Returns the K split (0: the block kernel takes the shape).
@@ -134,6 +136,7 @@ int nnq_rule_gemm_wide6(int64_t m, int64_t ntile, int64_t nblk) {
     const int64_t base = (m + 255) / 256 * (ntile / 8), n = ntile * 16;
     // the block kernel: 128-row tiles at about 350 TFLOP/s, its staging and slab sum 12 us
     float best = 12.0f + 2.0f * (float)((m + 127) / 128 * 128) * (float)n * (float)(nblk * 256) / 350.0e6f;
+    if (m <= 160) best *= 0.88f;
     int ks = 0;
     for (int split = 1; split <= 8; split++) {
         const int64_t wg = base * split;

@@ -113,3 +113,20 @@ def test_moe_few_is_a_limit_in_tokens(rules, experts, hidden, inter, top_k, bf16
 ])
 def test_few_rows_where_they_are_faster(rules, fmt, m, n, k, bf16, few):
     assert rules.few_rows(fmt, m, n, k, bf16) == few
+
+
+# Q6_K prefill measured on the block and the wide kernel (us, block / wide).
+@pytest.mark.parametrize("m,n,k,wide", [
+    (129, 40960, 1024, 0),   # 59.4 / 66.1
+    (160, 40960, 1024, 0),   # 62.1 / 66.9
+    (129, 9728, 2560, 0),    # 45.7 / 47.9
+    (200, 40960, 1024, 1),   # 74.6 / 67.6
+    (160, 12288, 4096, 2),   # 87.0 / 68.7
+    (129, 4096, 4096, 8),    # 35.3 / 31.5
+    (160, 6144, 2048, 4),    # 34.8 / 31.1
+    (129, 4096, 12288, 8),   # 74.3 / 56.2
+    (129, 24576, 1536, 1),   # 54.9 / 49.2
+    (512, 4096, 12288, 4),   # 133.8 / 103.6
+])
+def test_wide6_where_it_is_faster(rules, m, n, k, wide):
+    assert rules.wide6(m, n, k) == wide
