@@ -88,7 +88,10 @@ int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16) 
 // of whole super-blocks) are the ones with the least estimated time: rounds of workgroups over
 // the CUs, each 3 us and its super-blocks times the measured time of one (us, 6, 4 and 8 tiles: bf16 x
 // 3.8, 3.0 and 5.0, f32 x 6.2, 5.2 and 7.8: more tiles read each A fragment less often), plus
-// the slabs' write, read and launch.  512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles;
+// the slabs' write, read and launch.  With bf16 x a part of two super-blocks, whose prologue nothing
+// hides, counts as 2.7 and each further part adds 1.8% (without the two: 400 x 2560 x 2560 in 8 tiles and
+// K in five 27.9 us, in 4 tiles and K in two 25.0; 200 x 6144 x 2048 25.4 and 23.6; 129 x 8192 x 3072 28.7
+// and 26.6).  512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles;
 // the ring kernel over two planes 153) and 115 at 4096 x 12288 (8 tiles, K in four; 4 tiles
 // and K in two 134, ring 155), of bf16 x there 77 (4 tiles 83); 203 rows of f32 x at 12288 x
 // 4096 take 6 tiles and K in two (256 workgroups).
@@ -108,7 +111,12 @@ int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *
             const int64_t wg = nrt * (ntile / c) * split;
             if (wg < 128 || nblk % split || nblk / split < 2) continue;
             const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(m * n) * 4.0f / 4.0e6f : 0.0f;
-            const float us = (float)((wg + 255) / 256) * (3.0f + (float)(nblk / split) * sb_us[x_bf16 ? 0 : 1][i]) + slabs;
+            float sb = (float)(nblk / split), us = 1.0f;
+            if (x_bf16) {
+                sb = std::max(sb, 2.7f);
+                us = 1.0f + 0.018f * (float)(split - 1);
+            }
+            us *= (float)((wg + 255) / 256) * (3.0f + sb * sb_us[x_bf16 ? 0 : 1][i]) + slabs;
             if (!nt || us < best) {
                 best = us;
                 nt = c;

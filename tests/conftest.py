@@ -1,4 +1,5 @@
-"""Shared pytest setup: the `gpu` marker, repo root on sys.path, the oracle build."""
+"""Shared pytest setup: the `gpu` marker, repo root on sys.path, the oracle build, the dispatch rules."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -28,3 +29,36 @@ _ensure_oracle()
 def O():
     from oracle import oracle
     return oracle
+
+
+@pytest.fixture(scope="session")
+def rules():
+    """Which kernel a shape takes (nn_amd/csrc/nnq_plan.cpp)."""
+    from nn_amd import _lib
+    lib = _lib.load()
+    i64, c_int = ctypes.c_int64, ctypes.c_int
+    lib.nnq_rule_few_rows.argtypes = [c_int, i64, i64, i64, c_int]
+    lib.nnq_rule_gemm_wide.argtypes = [i64, i64, i64, c_int, ctypes.POINTER(c_int)]
+    lib.nnq_rule_gemm_wide6.argtypes = [i64, i64, i64]
+    lib.nnq_rule_moe_few.argtypes = [i64, i64, i64, i64, c_int, c_int]
+
+    class Rules:
+        @staticmethod
+        def few_rows(fmt, m, n, k, bf16):
+            return lib.nnq_rule_few_rows(fmt, (n + 15) // 16, k, m, bf16)
+
+        @staticmethod
+        def wide(m, n, k, bf16):
+            """(column tiles per workgroup, K split); (0, 0) where the wide Q4_K kernel does not take it"""
+            ks = c_int(0)
+            return lib.nnq_rule_gemm_wide(m, n // 16, k // 256, bf16, ctypes.byref(ks)), ks.value
+
+        @staticmethod
+        def wide6(m, n, k):
+            return lib.nnq_rule_gemm_wide6(m, n // 16, k // 256)
+
+        @staticmethod
+        def moe_few(experts, hidden, inter, tokens, top_k, bf16):
+            return lib.nnq_rule_moe_few(experts, hidden, inter, tokens, top_k, bf16)
+
+    return Rules

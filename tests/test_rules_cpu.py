@@ -1,44 +1,10 @@
 """The rules that choose a kernel by sizes alone (nn_amd/csrc/nnq_plan.cpp), asked through their C names:
 what holds for every shape.  No GPU needed."""
-import ctypes
 import random
 
 import pytest
 
 Q8_0, Q4_K, Q6_K = 8, 12, 14
-i64, c_int = ctypes.c_int64, ctypes.c_int
-
-
-@pytest.fixture(scope="module")
-def rules():
-    from nn_amd import _lib
-    lib = _lib.load()
-    lib.nnq_rule_few_rows.argtypes = [c_int, i64, i64, i64, c_int]
-    lib.nnq_rule_gemm_wide.argtypes = [i64, i64, i64, c_int, ctypes.POINTER(c_int)]
-    lib.nnq_rule_gemm_wide6.argtypes = [i64, i64, i64]
-    lib.nnq_rule_moe_few.argtypes = [i64, i64, i64, i64, c_int, c_int]
-
-    class Rules:
-        @staticmethod
-        def few_rows(fmt, m, n, k, bf16):
-            return lib.nnq_rule_few_rows(fmt, (n + 15) // 16, k, m, bf16)
-
-        @staticmethod
-        def wide(m, n, k, bf16):
-            """(column tiles per workgroup, K split); (0, 0) where the wide Q4_K kernel does not take it"""
-            ks = c_int(0)
-            return lib.nnq_rule_gemm_wide(m, n // 16, k // 256, bf16, ctypes.byref(ks)), ks.value
-
-        @staticmethod
-        def wide6(m, n, k):
-            return lib.nnq_rule_gemm_wide6(m, n // 16, k // 256)
-
-        @staticmethod
-        def moe_few(experts, hidden, inter, tokens, top_k, bf16):
-            return lib.nnq_rule_moe_few(experts, hidden, inter, tokens, top_k, bf16)
-
-    return Rules
-
 
 def test_kernel_limits(rules):
     """No rule sends a kernel what it cannot run: rows of the few-row GEMM, tiles and K parts that divide
@@ -130,3 +96,19 @@ def test_few_rows_where_they_are_faster(rules, fmt, m, n, k, bf16, few):
 ])
 def test_wide6_where_it_is_faster(rules, m, n, k, wide):
     assert rules.wide6(m, n, k) == wide
+
+
+# Q4_K prefill measured with other tiles and splits (us, what the rule takes / the other one named).
+@pytest.mark.parametrize("m,n,k,bf16,tiles,split", [
+    (400, 2560, 2560, 1, 4, 2),    # 25.0 / 27.9 with 8 tiles, K in five
+    (512, 2560, 2560, 1, 4, 2),    # 27.2 / 29.5 with 8 tiles, K in five
+    (200, 6144, 2048, 1, 4, 2),    # 23.6 / 25.4 with 6 tiles, K in four
+    (129, 8192, 3072, 1, 4, 2),    # 26.6 / 28.7 with 8 tiles, K in four
+    (768, 4096, 12288, 1, 8, 2),   # 109.6 / 118.6 with 8 tiles, K in eight
+    (512, 4096, 12288, 1, 8, 4),   # 69.0 / 77 with 4 tiles, K in two
+    (512, 4096, 12288, 0, 8, 4),   # 105.1 / 142.1 in the ring kernel
+    (203, 12288, 4096, 0, 6, 2),   # 57.9 / 74.0 in the ring kernel
+    (512, 24576, 4096, 1, 6, 1),
+])
+def test_wide_tiles_where_they_are_faster(rules, m, n, k, bf16, tiles, split):
+    assert rules.wide(m, n, k, bf16) == (tiles, split)
