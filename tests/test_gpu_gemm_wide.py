@@ -68,15 +68,9 @@ def test_wide_row_scales(O, dev):
     assert err.max() <= 1e-3
 
 
-# f32 activations (hi + lo planes) on the wide kernel: one row past its lower limit, ragged row
-# tiles, the three column-tile widths (the last three shapes: eight tiles, also for bf16), K split
-# two to four ways and not at all, K of the staging's limit.  Bar: max |error| <= 2e-5 of the output's rms: f32 sums over K <= 12288 of products
-# that keep 22 bits of x (2.3e-6 measured at 512 x 4096 x 12288).
-@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("m,n,k", [(129, 3072, 1024), (203, 12288, 512), (300, 6144, 2048), (513, 4096, 1280),
-                                   (256, 2048, 12288), (700, 1920, 768), (512, 4096, 2048), (1100, 4096, 512),
-                                   (1000, 2048, 2560)])
-def test_wide_activations(dev, m, n, k, xdt):
+def check_activations(dev, m, n, k, xdt):
+    """Bar: max |error| <= 2e-5 of a row's rms: f32 sums over K <= 12288 of products that keep 22 bits of x
+    (2.3e-6 measured at 512 x 4096 x 12288)."""
     import nn_amd
     w = make_weight("q4_k", nn_amd.quantize_q4_k(nn_amd.synth_normal(m, 1, (n, k), 0.02)), n, k)
     x = torch.from_numpy(nn_amd.synth_normal(m, 2, (m, k), 1.0)).to(dev)
@@ -93,13 +87,55 @@ def test_wide_activations(dev, m, n, k, xdt):
     assert torch.equal(yb, y.to(torch.bfloat16)), "bf16 output: the f32 result rounded once"
 
 
+# f32 and bf16 activations from the wide kernel's lower limit on, ragged row tiles, K up to the
+# staging's limit.  (129 x 3072 x 1024 and 700 x 1920 x 768 are too few workgroups for the wide kernel:
+# the ring kernel at the same row counts.)
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(129, 3072, 1024), (203, 12288, 512), (300, 6144, 2048), (513, 4096, 1280),
+                                   (256, 2048, 12288), (700, 1920, 768), (512, 4096, 2048), (1100, 4096, 512),
+                                   (1000, 2048, 2560)])
+def test_wide_activations(dev, m, n, k, xdt):
+    check_activations(dev, m, n, k, xdt)
+
+
+# Every instantiation of the wide kernel, with and without a K split: one row past the lower limit, a row
+# past one and two row tiles; parts of two super-blocks (the fewest), and of three and more, where the
+# ring of min-term operands wraps.  The rule has to give the tiles and the split named here.
+@pytest.mark.parametrize("xdt,m,n,k,tiles,split", [
+    ("f32", 129, 1024, 4096, 4, 8), ("f32", 257, 4096, 512, 4, 1), ("f32", 513, 6144, 512, 6, 1),
+    ("f32", 257, 3072, 1536, 6, 3), ("f32", 203, 6144, 4096, 6, 4), ("f32", 513, 8192, 512, 8, 1),
+    ("f32", 513, 4096, 2048, 8, 2), ("f32", 257, 2048, 2560, 8, 5), ("bf16", 129, 1024, 4096, 4, 8),
+    ("bf16", 257, 4096, 1280, 4, 1), ("bf16", 257, 2048, 2048, 4, 4), ("bf16", 513, 6144, 512, 6, 1),
+    ("bf16", 257, 3072, 3072, 6, 4), ("bf16", 513, 8192, 512, 8, 1), ("bf16", 513, 3072, 3072, 8, 3),
+    ("bf16", 513, 2048, 4096, 8, 4)])
+def test_wide_tiles_and_splits(dev, rules, xdt, m, n, k, tiles, split):
+    assert rules.wide(m, n, k, xdt == "bf16") == (tiles, split)
+    check_activations(dev, m, n, k, torch.bfloat16 if xdt == "bf16" else torch.float32)
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [(129, 1024, 4096, 4), (203, 6144, 4096, 6), (513, 4096, 2048, 8)])
+def test_wide_f32_random_blocks(O, dev, rules, m, n, k, tiles):
+    """Random block bytes (any finite d, dmin and scales) with f32 x, whose codes the kernel forms as
+    normal f16 numbers; bars of test_gpu_linear."""
+    import nn_amd
+    assert rules.wide(m, n, k, 0)[0] == tiles
+    b = rand_bytes("q4_k", n, k, seed=m + n + k).reshape(-1, 144).copy()
+    b[::7, 0:2] = 0  # d = +0.0 for every seventh super-block
+    b = b.ravel()
+    w = make_weight("q4_k", b, n, k)
+    x = nn_amd.synth_normal(m + 1, 2, (m, k), 1.0)
+    y = nn_amd.quantized_linear(torch.from_numpy(x).to(dev), w).cpu().numpy()
+    check_close(ref_f64(O, b, n, k, x), y, f"gemm wide f32 {m}x{n}x{k}")
+
+
 @pytest.mark.parametrize("m,hidden,inter,xdt", [(129, 512, 6144, torch.bfloat16), (300, 1024, 3072, torch.float32),
                                                (600, 512, 2048, torch.bfloat16)])
-def test_prefill_mlp_swiglu_epilogue(dev, m, hidden, inter, xdt):
+def test_prefill_mlp_swiglu_epilogue(dev, rules, m, hidden, inter, xdt):
     """The gate | up GEMM that writes silu(gate) * up itself, against the three linears: h differs by
     f32 rounding only, so the outputs agree to 1e-5 of their rms; a NaN row is flagged and stays
     in its row."""
     import nn_amd
+    assert rules.wide(m, 2 * inter, hidden, xdt == torch.bfloat16)[1] == 1  # the wide kernel, K not split
     q = [nn_amd.quantize_q4_k(nn_amd.synth_normal(5, i, s, 0.02))
          for i, s in ((1, (inter, hidden)), (2, (inter, hidden)), (3, (hidden, inter)))]
     mlp = nn_amd.QuantizedMLP(*q, nn_amd.QuantType.Q4_K, hidden, inter)
