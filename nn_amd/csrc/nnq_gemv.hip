@@ -1,5 +1,4 @@
-// Decode GEMV (up to 8 tokens per launch: Q4_K and Q6_K 4, Q8_0 8) for Q4_K / Q8_0 / Q6_K
-// weights on gfx950.
+// Decode GEMV (up to 4 tokens per launch) for Q4_K / Q8_0 / Q6_K weights on gfx950.
 //
 // One workgroup owns a tile of 16 weight rows.  Its waves split K into units (256
 // elements; 8 blocks for Q8_0) and issue the activation slices and the weight loads of
@@ -1107,9 +1106,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_decode_kernel(const uint8
 // per-wave LDS table (8 powers of two and 8 sums per token) that each lane group reads
 // for its two tokens with broadcast 16-byte reads.  One unit per wave and pass.
 // ---------------------------------------------------------------------------------
-template <int WAVES, int XM, int MT>
+template <int WAVES, bool XB>
 __global__ __launch_bounds__(WAVES * 64) void gemv_q80_batch_kernel(GemvArgs a) {
-    constexpr bool XB = XM == 1;
+    constexpr int MT = 4;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = (int)blockIdx.x, mt = (int)a.m;
@@ -1127,25 +1126,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_batch_kernel(GemvArgs a) 
     const uint8_t *qbase = a.qs + (size_t)tile * (size_t)(a.nblk / 2) * 1024 + 16 * lane;
     const uint8_t *hbase = a.hdr + (size_t)tile * units * 256 + 16 * r16;
     constexpr int xe = XB ? 2 : 4;
-    const int xrow = XM == 2 ? 2 * k : k;
     const uint8_t *xb = reinterpret_cast<const uint8_t *>(a.x);
     float acc1[2] = {0.f, 0.f}, acc2[2] = {0.f, 0.f};
     for (int ub0 = 0; ub0 < units; ub0 += WAVES) {
         const int u = min(ub0 + wv, units - 1);
         const int kk = u * 256 + 4 * lane;
         const bool xin = kk < k;
-        u32x4 xr[MT], xu[XM == 2 ? MT : 1];
+        u32x4 xr[MT];
 #pragma unroll
         for (int t = 0; t < MT; t++) {
             const bool tin = xin && t < mt;
-            const uint8_t *p = xb + (size_t)(tin ? t * xrow + kk : 0) * xe;  // out of range: x[0]
+            const uint8_t *p = xb + (size_t)(tin ? t * k + kk : 0) * xe;  // out of range: x[0]
             if (XB) {
                 const u32x2 w2 = *reinterpret_cast<const u32x2 *>(p);
                 xr[t] = u32x4{w2[0], w2[1], 0u, 0u};
             } else {
                 xr[t] = *reinterpret_cast<const u32x4 *>(p);
             }
-            if constexpr (XM == 2) xu[t] = *reinterpret_cast<const u32x4 *>(p + (size_t)k * 4);
         }
         __builtin_amdgcn_sched_barrier(0);  // keep this issue order
         UnitQ80 w;
@@ -1156,10 +1153,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_batch_kernel(GemvArgs a) 
         if (ub0 + wv >= units) break;  // wave-uniform: no unit left for this wave
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            u32x4 xv = xr[t];
-            if constexpr (XM == 2) xv = swiglu4(xv, xu[t]);
             float bk, xs;
-            stage_q80<XB>(xv, xin && t < mt, xbuf[wv] + 512 * t, xbuf[wv] + 512 * t + 256, bk, xs);
+            stage_q80<XB>(xr[t], xin && t < mt, xbuf[wv] + 512 * t, xbuf[wv] + 512 * t + 256, bk, xs);
             if ((lane & 7) == 0) {
                 stats[wv][t][lane >> 3] = bk;
                 stats[wv][t][8 + (lane >> 3)] = xs;
@@ -1933,14 +1928,11 @@ static int launch_q80_decode_t(const GemvArgs &a, void *stream) {
 }
 template <int WAVES>
 static int launch_q80_batch_t(const GemvArgs &a, void *stream) {
-    if (a.x_swiglu)
-        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 2, 4>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
-                           (hipStream_t)stream, a);
-    else if (a.x_bf16)
-        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 1, 4>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
+    if (a.x_bf16)
+        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, true>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
                            (hipStream_t)stream, a);
     else
-        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, 0, 4>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
+        hipLaunchKernelGGL((gemv_q80_batch_kernel<WAVES, false>), dim3((unsigned)a.ntile), dim3(WAVES * 64), 0,
                            (hipStream_t)stream, a);
     return (int)hipGetLastError();
 }
@@ -2103,10 +2095,10 @@ static int launch_q4k_decode(const GemvArgs &a, void *stream) {
     return launch_q4k_decode_t<16, 4>(a, stream);
 }
 
-// tokens per launch: Q4_K and Q6_K up to 4, Q8_0 up to 8 (callers run passes)
+// tokens per launch: up to 4, the batch kernels' token rows (callers run passes); a SwiGLU input or
+// output up to 2
 int launch_gemv(int fmt, const GemvArgs &a, void *stream) {
-    const int mmax = fmt == FQ80 ? 8 : 4;
-    if (a.m < 1 || a.m > mmax) return (int)hipErrorInvalidValue;
+    if (a.m < 1 || a.m > 4 || (a.m > 2 && (a.x_swiglu || a.swiglu_out))) return (int)hipErrorInvalidValue;
     const int64_t units = fmt == FQ80 ? a.nblk / 8 : a.nblk;
     switch (fmt) {
     case FQ4K: return launch_q4k_decode(a, stream);

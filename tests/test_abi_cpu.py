@@ -182,3 +182,26 @@ def test_ocp_mxfp4_encoder_matches_oracle(O):
         assert np.array_equal(nn_amd.quantize_mxfp4_ocp(v), O.ocp_quantize(v)), scale
     with pytest.raises(nn_amd.NonFiniteData):
         nn_amd.quantize_mxfp4_ocp(np.array([0.0, np.inf], np.float32))
+
+
+def test_gemv_launch_refuses_more_tokens_than_its_kernels_hold(lib):
+    """The GEMV launch (GemvArgs, nn_amd/csrc/nnq_internal.h) is an internal entry; a caller's mistake in its
+    tokens has to come back as an error and not as rows of another wave's sums.  Every refused count
+    returns before a launch, so no GPU is touched."""
+    class GemvArgs(ctypes.Structure):
+        _fields_ = [("qs", ctypes.c_void_p), ("hdr", ctypes.c_void_p), ("x", ctypes.c_void_p), ("x_bf16", ctypes.c_int),
+                    ("bias", ctypes.c_void_p), ("y", ctypes.c_void_p), ("y_bf16", ctypes.c_int), ("n", ctypes.c_int64),
+                    ("k", ctypes.c_int64), ("m", ctypes.c_int64), ("ntile", ctypes.c_int64), ("nblk", ctypes.c_int64),
+                    ("kc", ctypes.c_int), ("logits_out", ctypes.c_void_p), ("argmax_partial", ctypes.c_void_p),
+                    ("argmax_count", ctypes.c_void_p), ("x_swiglu", ctypes.c_int), ("swiglu_out", ctypes.c_int),
+                    ("status", ctypes.c_void_p), ("status_mode", ctypes.c_int)]
+
+    launch = lib._ZN3nnq11launch_gemvEiRKNS_8GemvArgsEPv
+    launch.argtypes = [ctypes.c_int, ctypes.POINTER(GemvArgs), ctypes.c_void_p]
+    invalid = 1  # hipErrorInvalidValue
+    for fmt in (8, 12, 14):
+        for m in (-1, 0, 5, 6, 8, 9, 1 << 33):
+            assert launch(fmt, ctypes.byref(GemvArgs(n=16, k=256, m=m, ntile=1, nblk=8)), None) == invalid, (fmt, m)
+        for kind in ("x_swiglu", "swiglu_out"):
+            a = GemvArgs(n=16, k=256, m=3, ntile=1, nblk=8, **{kind: 1})
+            assert launch(fmt, ctypes.byref(a), None) == invalid, (fmt, kind)
