@@ -380,6 +380,34 @@ def test_argmax_semantics(dev):
         nn_amd.argmax(v)
 
 
+@pytest.mark.parametrize("n,k", [(37, 512), (30000, 512)])
+def test_linear_argmax_index_types(dev, n, k):
+    """The C entry points with a 32-bit and with a 64-bit index give the same logits, index and status
+    (one tile a workgroup, and the streaming kernel's one key a workgroup), and write nothing beside
+    the index; a NaN logit gives index 0 and its status."""
+    import nn_amd
+    from nn_amd import _lib
+    lib = _lib.load()
+    w = make_weight("q6_k", nn_amd.quantize_q6_k(nn_amd.synth_normal(51, 1, (n, k), 0.02)), n, k)
+    x = torch.from_numpy(nn_amd.synth_normal(51, 2, (k,), 1.0)).to(dev)
+    for nan in (False, True):
+        if nan:
+            x[3] = float("nan")
+        got = []
+        for call, dt in ((lib.nnq_linear_argmax, torch.int32), (lib.nnq_linear_argmax_i64, torch.int64)):
+            logits = torch.zeros(n, device=dev)
+            idx, st = torch.full((3,), -7, dtype=dt, device=dev), torch.full((3,), -7, dtype=torch.int32, device=dev)
+            rc = call(w.handle, x.data_ptr(), k, None, 0, logits.data_ptr(), idx[1:].data_ptr(), st[1:].data_ptr(),
+                      torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, _lib.last_error()
+            assert idx.tolist()[::2] == [-7, -7] and st.tolist()[::2] == [-7, -7]
+            got.append((logits, int(idx[1]), int(st[1])))
+        assert torch.equal(got[0][0].view(torch.int32), got[1][0].view(torch.int32)) and got[0][1:] == got[1][1:]
+        assert got[0][1:] == ((0, _lib.ERR_NON_FINITE) if nan else (int(got[0][0].argmax()), 0))
+        rc = lib.nnq_linear_argmax(w.handle, x.data_ptr(), k, None, 0, logits.data_ptr(), None, None, None)
+        assert rc == _lib.ERR_INVALID_ARGUMENT  # no index
+
+
 def test_lm_head_argmax_graph_replay(O, dev):
     """The streaming LM head (one argmax key per workgroup, then argmax_final_kernel)
     captured into a HIP graph: every replay, and eager calls with another input between
