@@ -344,7 +344,9 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *logits, int
 
 // Routing for E > 256 experts: the same computation as moe_route_kernel with the
 // token's values in LDS (one row of E floats per wave, dynamic shared memory); the
-// selection rounds mark a chosen expert by key 0 (every probability key is above it).
+// selection rounds mark a chosen expert by key 0.  Every probability's key is above it: that of
+// the NaN with all bits set, the least of all, is raised to 1 (a token whose probabilities were
+// all this NaN found no expert, wrote past the keys and left its rows' places unwritten).
 __global__ __launch_bounds__(256) void moe_route_any_kernel(const float *logits, int nsplit, const float *bias,
                                                             int64_t T, int E, int k, uint32_t *ti, float *tw,
                                                             uint32_t *ti_out, float *tw_out) {
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(256) void moe_route_any_kernel(const float *logits,
     uint32_t idx[8];
     float val[8];
     float ssum = -0.0f;
-    for (int c = lane; c < E; c += 64) key[c] = (uint32_t)total_key(v[c]) ^ 0x80000000u;
+    for (int c = lane; c < E; c += 64) key[c] = max((uint32_t)total_key(v[c]) ^ 0x80000000u, 1u);
     wave_sync();
     for (int s = 0; s < k; s++) {
         uint64_t best = 0;

@@ -489,3 +489,28 @@ def test_moe_many_rows_per_expert(O, dev, E, H, I, T, k, xdt, skew):
     ref, rti, rtw = O.moe_forward(x.float().cpu().numpy(), lg, k, L["gp"], L["gs"], L["gb"], L["dp"], L["ds"], L["db"], I)
     assert np.array_equal(ti.cpu().numpy().astype(np.uint32), rti), "routing differs"
     check_close(ref, y.cpu().numpy(), f"moe many rows E={E} T={T} k={k} x={xdt} skew={skew}")
+
+
+@pytest.mark.parametrize("E,T,k", [(300, 5, 4), (300, 40, 9), (300, 1030, 2), (32, 5, 4), (32, 40, 9)])
+def test_moe_routing_nan_logits(O, dev, E, T, k):
+    """A NaN logit of any bit pattern, all bits set among them, gives its token NaN weights over distinct
+    experts of the layer and leaves the other tokens' routing and outputs as they are."""
+    import nn_amd
+    H, I = 64, 32
+    L = make_layer(E, H, I, seed=E + T)
+    moe = upload(L, E, H, I)
+    x = torch.from_numpy(nn_amd.synth_normal(37, 5, (T, H), 1.0)).to(dev)
+    lg = nn_amd.synth_normal(37, 6, (T, E), 2.0)
+    good, ti, tw = moe.forward(x, torch.from_numpy(lg).to(dev), top_k=k, return_routing=True)
+    bits = lg.view(np.uint32)
+    bad = {0: 0xFFFFFFFF, 2: 0x7FC00000, 3: 0xFFC00000, T - 1: 0xFFFFFFFF}
+    for t, b in bad.items():
+        bits[t, (7 * t) % E] = b
+    y, ti2, tw2 = moe.forward(x, torch.from_numpy(lg).to(dev), top_k=k, return_routing=True)
+    rows = list(bad)
+    keep = torch.ones(T, dtype=torch.bool)
+    keep[rows] = False
+    assert torch.equal(y[keep.to(dev)], good[keep.to(dev)]) and torch.equal(ti2[keep.to(dev)], ti[keep.to(dev)])
+    assert torch.isnan(tw2[rows]).all() and torch.isnan(y[rows]).all()
+    for r in ti2[rows].cpu().numpy().astype(np.int64):
+        assert len(set(r)) == k and r.min() >= 0 and r.max() < E
