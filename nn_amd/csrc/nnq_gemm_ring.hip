@@ -430,44 +430,12 @@ int launch_rk(const GemmArgs &a, const GemmScratch &sc, hipStream_t st) {
 
 }  // namespace
 
-// Shapes the ring kernel takes (N % 128 == 0, a 16-byte aligned output; f32 activations run
-// their staged hi and lo planes as two halves of the work, summed by the finalize):
-// BM x BN tiles, BM the smallest of 32, 64, 128 holding M (128 beyond), BN 192 or 128
-// (dividing N), K split 1, 2, 4, 8 or 16 ways (a divisor of the super-block count leaving
-// at least 4 super-blocks per workgroup, 2 with BM < 128).  Of these, the plan with the
-// least estimated time: rounds of workgroups (one resident per CU: the rings of the small
-// row tiles are deepened to 6 stages, which LDS holds once) times stages per workgroup, a 128-wide
-// stage at 0.8 of a 192-wide one, plus one stage for the split-K finalize.  (Assuming two
-// resident workgroups with shallower rings measured 5-25% slower at M = 16 to 64.)
-// Returns the K split, or 0 when the shape does not fit.
+// The ring kernel's K split (0: the shape does not fit) and tile: the rule of its shape
+// (nnq_rule_gemm_ring), for whole 16-row weight tiles and a 16-byte aligned output (the output tile is
+// written in 16-byte chunks of whole rows).
 int gemm_ring_plan(const GemmArgs &a, int *bn, int *bm) {
-    // (the output tile is written in 16-byte chunks of whole rows: no partial last tile)
-    if (a.m < 1 || a.nblk < 1 || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
-    const int npl = a.x_bf16 ? 1 : 2;  // f32 activations: hi and lo planes, each a full pass
-    const int rows = a.m <= 32 ? 32 : (a.m <= 64 ? 64 : 128);
-    const int64_t ncols = a.ntile * 16, nrt = (a.m + rows - 1) / rows;
-    const int min_sb = rows == 128 ? 4 : 2, per_cu = 1;
-    double best_cost = 0.0;
-    int best_bn = 0, best_ks = 0;
-    for (int cand : {192, 128}) {
-        if (ncols % cand) continue;
-        for (int ks = 1; ks <= 16; ks *= 2) {
-            if (a.nblk % ks || (ks > 1 && a.nblk / ks < min_sb)) continue;
-            const int64_t wgs = nrt * (ncols / cand) * ks * npl;
-            const int64_t rounds = (wgs + 256 * per_cu - 1) / (256 * per_cu);
-            const double cost =
-                (double)rounds * (double)(a.nblk / ks) * (cand == 192 ? 1.0 : 0.8) + (ks * npl > 1 ? 1.0 : 0.0);
-            if (best_bn == 0 || cost < best_cost) {
-                best_cost = cost;
-                best_bn = cand;
-                best_ks = ks;
-            }
-        }
-    }
-    if (best_bn == 0) return 0;
-    if (bn) *bn = best_bn;
-    if (bm) *bm = rows;
-    return best_ks;
+    if (a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
+    return nnq_rule_gemm_ring(a.m, a.ntile, a.nblk, a.x_bf16, bn, bm);
 }
 
 int launch_gemm_finalize(const float *ys, int ks, const float *bias, void *y, int y_bf16, int64_t m, int64_t n,

@@ -80,6 +80,7 @@ constexpr int kMoeFewT = 16;        // moe_few_kernel: most tokens
 constexpr int kMoeFewAssign = 128;  //   and assignments (two per lane of its ballots)
 extern "C" {
 int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16);  // 1: gemm_few_kernel
+int nnq_rule_gemm_ring(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *bn, int *bm);
 int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *ks);
 int nnq_rule_gemm_wide6(int64_t m, int64_t ntile, int64_t nblk);
 int nnq_rule_moe_few(int64_t experts, int64_t hidden, int64_t inter, int64_t tokens, int top_k, int x_bf16);
@@ -169,7 +170,8 @@ int launch_gemm_thin(const GemmArgs &a, void *stream);
 int gemm_few_rows(int fmt);
 size_t gemm_few_scratch_bytes(const GemmArgs &a, int fmt);
 int launch_gemm_few(const GemmArgs &a, int fmt, void *stream);
-// Q8_0 / Q6_K prefill GEMM (M > 8): the activation staging below, then one kernel
+// Q8_0 / Q6_K prefill GEMM (what nnq_rule_few_rows leaves, from M = 5 on): the activation staging
+// below, then one kernel
 int launch_gemm_blk(const GemmArgs &a, void *stream);
 // its K split (and tile height and width, when bm / bn are given)
 int gemm_blk_plan(const GemmArgs &a, int *bm, int *bn = nullptr);

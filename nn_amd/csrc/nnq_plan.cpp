@@ -80,6 +80,43 @@ int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16) 
     return m > 6 || (m > 4 && (ntile >= 512 || k > 8192));
 }
 
+// Shapes the Q4_K ring kernel takes (N % 128 == 0; f32 activations run their staged hi and lo
+// planes as two halves of the work, summed by the finalize):
+// BM x BN tiles, BM the smallest of 32, 64, 128 holding M (128 beyond), BN 192 or 128
+// (dividing N), K split 1, 2, 4, 8 or 16 ways (a divisor of the super-block count leaving
+// at least 4 super-blocks per workgroup, 2 with BM < 128).  Of these, the plan with the
+// least estimated time: rounds of workgroups (one resident per CU: the rings of the small
+// row tiles are deepened to 6 stages, which LDS holds once) times stages per workgroup, a 128-wide
+// stage at 0.8 of a 192-wide one, plus one stage for the split-K finalize.  (Assuming two
+// resident workgroups with shallower rings measured 5-25% slower at M = 16 to 64.)
+// Returns the K split, or 0 when the shape does not fit.
+int nnq_rule_gemm_ring(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *bn, int *bm) {
+    if (m < 1 || nblk < 1) return 0;
+    const int npl = x_bf16 ? 1 : 2;  // f32 activations: hi and lo planes, each a full pass
+    const int rows = m <= 32 ? 32 : (m <= 64 ? 64 : 128);
+    const int64_t ncols = ntile * 16, nrt = (m + rows - 1) / rows;
+    const int min_sb = rows == 128 ? 4 : 2;
+    double best_cost = 0.0;
+    int best_bn = 0, best_ks = 0;
+    for (int cand : {192, 128}) {
+        if (ncols % cand) continue;
+        for (int ks = 1; ks <= 16; ks *= 2) {
+            if (nblk % ks || (ks > 1 && nblk / ks < min_sb)) continue;
+            const int64_t rounds = (nrt * (ncols / cand) * ks * npl + 255) / 256;
+            const double cost = (double)rounds * (double)(nblk / ks) * (cand == 192 ? 1.0 : 0.8) + (ks * npl > 1 ? 1.0 : 0.0);
+            if (best_bn == 0 || cost < best_cost) {
+                best_cost = cost;
+                best_bn = cand;
+                best_ks = ks;
+            }
+        }
+    }
+    if (best_bn == 0) return 0;
+    if (bn) *bn = best_bn;
+    if (bm) *bm = rows;
+    return best_ks;
+}
+
 // The wide kernel's shape rules: more than 128 rows (below, half of a 256-row tile or more is
 // padding: f32 x, 100 x 4096 x 12288 109 us against the ring's 51), whole 16-row weight tiles
 // and a 16-byte aligned output (the epilogue writes 16-byte row chunks), K <= 4096 * 3 (the
