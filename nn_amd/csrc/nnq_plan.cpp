@@ -128,40 +128,57 @@ int nnq_rule_gemm_ring(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *
 // the slabs' write, read and launch.  With bf16 x a part of two super-blocks, whose prologue nothing
 // hides, counts as 2.7 and each further part adds 1.8% (without the two: 400 x 2560 x 2560 in 8 tiles and
 // K in five 27.9 us, in 4 tiles and K in two 25.0; 200 x 6144 x 2048 25.4 and 23.6; 129 x 8192 x 3072 28.7
-// and 26.6).  512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles;
-// the ring kernel over two planes 153) and 115 at 4096 x 12288 (8 tiles, K in four; 4 tiles
-// and K in two 134, ring 155), of bf16 x there 77 (4 tiles 83); 203 rows of f32 x at 12288 x
-// 4096 take 6 tiles and K in two (256 workgroups).
+// and 26.6).
+// 512 rows of f32 x take 107 us at 12288 x 4096 (6 tiles; the ring kernel over two planes 153) and
+// 115 at 4096 x 12288 (8 tiles, K in four; 4 tiles and K in two 134, ring 155), of bf16 x there 77
+// (4 tiles 83); 203 rows of f32 x at 12288 x 4096 take 6 tiles and K in two (256 workgroups).
 // With random x these rates are the chip's power limit for f16 products: a library f16 GEMM
 // of 512 x 12288 x 4096 takes 58 us (44 with x = 0), this kernel 66 with its staging (60).
+// With f32 x the ring kernel keeps what it does faster, above all K of a prime number of super-blocks,
+// which cannot be split here (260 x 5376 x 11008 125 us there, 187 here; 384 x 4736 x 1792 34 and 39).
+// Both sides' times are estimated with constants fitted to 288 calls of the ring and 713 of this
+// kernel, 4% and 5% off in the mean: us, per million of x, per MB of slabs (the ring's two planes have
+// one each), per round and per super-block of a round (the ring's 128-column tiles 0.8 of its wide ones).
 // Returns the column tiles per workgroup (0: the ring kernel takes the shape) and the K split.
 int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *ks) {
     if (m <= 128 || nblk > 48) return 0;
     const int64_t nrt = (m + 255) / 256, n = ntile * 16;
+    const int tiles[3] = {6, 4, 8};
     const float sb_us[2][3] = {{3.8f, 3.0f, 5.0f}, {6.2f, 5.2f, 7.8f}};
+    const float y_mb = (float)(m * n) * 4.0e-6f;
     float best = 0.0f;
-    int nt = 0;
+    int at = -1, best_ks = 0;
     for (int i = 0; i < 3; i++) {
-        const int c = i == 0 ? 6 : i == 1 ? 4 : 8;
-        if (ntile % c) continue;
+        if (ntile % tiles[i]) continue;
         for (int split = 1; split <= 8; split++) {
-            const int64_t wg = nrt * (ntile / c) * split;
+            const int64_t wg = nrt * (ntile / tiles[i]) * split;
             if (wg < 128 || nblk % split || nblk / split < 2) continue;
-            const float slabs = split > 1 ? 3.0f + (float)(split + 1) * (float)(m * n) * 4.0f / 4.0e6f : 0.0f;
-            float sb = (float)(nblk / split), us = 1.0f;
-            if (x_bf16) {
-                sb = std::max(sb, 2.7f);
-                us = 1.0f + 0.018f * (float)(split - 1);
-            }
-            us *= (float)((wg + 255) / 256) * (3.0f + sb * sb_us[x_bf16 ? 0 : 1][i]) + slabs;
-            if (!nt || us < best) {
+            const float sb = x_bf16 ? std::max((float)(nblk / split), 2.7f) : (float)(nblk / split);
+            float us = (float)((wg + 255) / 256) * (3.0f + sb * sb_us[x_bf16 ? 0 : 1][i]);
+            if (split > 1) us += 3.0f + (float)(split + 1) * y_mb * 0.25f;
+            if (x_bf16) us *= 1.0f + 0.018f * (float)(split - 1);
+            if (at < 0 || us < best) {
                 best = us;
-                nt = c;
-                if (ks) *ks = split;
+                at = i;
+                best_ks = split;
             }
         }
     }
-    return nt;
+    if (at < 0) return 0;
+    int bn = 0;
+    const int rks = x_bf16 ? 0 : nnq_rule_gemm_ring(m, ntile, nblk, 0, &bn, nullptr);
+    if (rks) {
+        const float x_m = (float)m * (float)(nblk * 256) * 1.0e-6f, f32_us[3] = {4.7f, 3.9f, 5.8f};
+        const int64_t rounds = (nrt * (ntile / tiles[at]) * best_ks + 255) / 256;
+        const int64_t rrounds = ((m + 127) / 128 * (n / bn) * rks * 2 + 255) / 256;
+        const float slabs = best_ks > 1 ? 0.5f + 0.22f * (float)(best_ks + 1) * y_mb : 0.0f;
+        const float wide = 7.1f + 1.37f * x_m + (float)rounds * (3.8f + (float)(nblk / best_ks) * f32_us[at]) + slabs;
+        const float ring = 10.4f + 1.05f * x_m + 0.34f * (float)(2 * rks + 1) * y_mb +
+                           3.15f * (float)(rrounds * (nblk / rks)) * (bn == 192 ? 1.0f : 0.8f);
+        if (ring < wide) return 0;
+    }
+    if (ks) *ks = best_ks;
+    return tiles[at];
 }
 
 // The wide Q6_K kernel's shape rules: bf16 activations, more than 128 rows, whole groups of 8 weight tiles, K up

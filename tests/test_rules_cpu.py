@@ -109,6 +109,12 @@ def test_wide6_where_it_is_faster(rules, m, n, k, wide):
     (512, 4096, 12288, 0, 8, 4),   # 105.1 / 142.1 in the ring kernel
     (203, 12288, 4096, 0, 6, 2),   # 57.9 / 74.0 in the ring kernel
     (512, 24576, 4096, 1, 6, 1),
+    (260, 5376, 11008, 0, 0, 0),   # ring kernel 124.6 / 186.9 with 4 tiles (43 super-blocks cannot be split)
+    (384, 5376, 11008, 0, 0, 0),   # ring kernel 127.0 / 188.0
+    (600, 5376, 11008, 0, 4, 1),   # 194.8 / 231.4 in the ring kernel
+    (384, 4736, 1792, 0, 0, 0),    # ring kernel 34.1 / 39.2 with 4 tiles
+    (600, 4736, 1792, 0, 4, 1),    # 40.8 / 54.8 in the ring kernel
+    (260, 5376, 11008, 1, 4, 1),   # 108.5 / 119.5 in the ring kernel
 ])
 def test_wide_tiles_where_they_are_faster(rules, m, n, k, bf16, tiles, split):
     assert rules.wide(m, n, k, bf16) == (tiles, split)
