@@ -1,4 +1,5 @@
-// Prefill GEMM for Q8_0 and Q6_K weights on gfx950 (M > 8 tokens):
+// Prefill GEMM for Q8_0 and Q6_K weights on gfx950 (more than 16 tokens, and 9 to 16 of Q6_K over
+// many tiles of short K; nnq_rule_few_rows):
 // Y[m, n] = X[m, k] . W[n, k]^T (+ bias), f32 accumulation, f32 or bf16 output: the
 // arithmetic of QLinear::forward with a batch of tokens for these formats
 // (crates/nn-core/src/layers/quantized/linear.rs:366-400; quantized_matmul_core,

@@ -1,7 +1,8 @@
 // GEMM over a few token rows on gfx950, Y[m, n] = X[m, k] . W[n, k]^T (+ bias), in one launch
 // that reads the weight once: Q8_0 and Q4_K weights for up to 16 rows of f32 or bf16 x, Q6_K
 // for up to 8 (quantized_linear over a served batch, crates/nn-core/src/dyn_tensor/
-// quantized_matmul.rs:367-406).  The weight is the decode GEMVs' tile16 image.
+// quantized_matmul.rs:367-406); 9 to 16 rows of Q6_K are two launches, which read the weight
+// twice.  The weight is the decode GEMVs' tile16 image.
 //
 // Bound: the weight stream from HBM (an LM head of 151936 x 4096 in Q6_K: 511 MB, 73 us), and
 // close behind it the VALU that forms the MFMA's B operands and applies the block scales, so
@@ -29,6 +30,8 @@
 // -> 97, 16 rows 271 -> 204 (two launches); Q8_0 4096 x 4096, 12 bf16 rows 17.3 -> 7.8;
 // Q4_K 4096 x 12288, 6 f32 rows 18.3 -> 16.0 (K split three ways), 12288 x 4096, 16 f32 rows
 // 27.3 -> 18.0.
+// Registers: 16 waves leave 128 each, which the f32 plane form (9 to 16 rows) passes by 6 (Q4_K)
+// and 10 (Q8_0), spilled; the other forms fit.
 // Rows: Q8_0 and Q4_K have one scale per 32 k, one MFMA row per token.  A Q6_K scale covers 16 k,
 // so token t takes rows 2t and 2t + 1, each with zeros in the other sub-block's half of k.
 // A NaN or infinity in a token's unit makes that token's outputs NaN.

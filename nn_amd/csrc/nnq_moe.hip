@@ -1457,10 +1457,12 @@ static int launch_stream_t(const MoeDev &d, const MoeScratch &sc, const MoeRun &
         attr_set = true;
     }
     // One slot while an expert has up to 64 rows on average (a slot without a pass still starts a
-    // workgroup), then enough for half again the average, at most 4 (more cost what they give:
-    // 2048 tokens of 32 experts of 2048 x 2048 576 us with 1, 511 with 2, 498 with 4, 527 with
-    // 5).  400 tokens on 16 experts 291 -> 174 us, 1000 f32 tokens on 8 of 2880 x 1440 566 ->
-    // 232; 32 experts of 2880 x 2880, whose one set already fills the chip, within 1%.
+    // workgroup), then enough for half again the average, at most 4.  Where one set leaves CUs
+    // idle the slots give 2 to 3 times (600 tokens, top 2 of 8 experts of 2880 x 2880 382 -> 150 us);
+    // where it fills the chip they are for uneven routing (2048 tokens with expert offsets N(0, 1):
+    // 32 experts of 2880 x 2880, top 4, 2725 -> 1235, 64 of 1440 x 1440, top 8, 1590 -> 806) and cost
+    // evenly loaded experts up to 4% (32 of 2880 x 2880, 600 tokens 265 -> 270, 2048 level), 9% at the
+    // worst (64 of 1440 x 1440, top 8, 1024 tokens 341 -> 373).
     const int64_t avg = run.A / d.E;
     const int64_t slots = avg <= 64 ? 1 : std::min<int64_t>(4, (avg + avg / 2 + 63) / 64);
     hipLaunchKernelGGL((moe_stream_kernel<P, GU, CKB, SL>), dim3((unsigned)(d.E * kMoeGroups * slots)),

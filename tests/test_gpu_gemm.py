@@ -1,4 +1,4 @@
-"""GPU parity for the Q4_K prefill GEMM (m > 8 tokens).
+"""GPU parity for the Q4_K GEMMs of more than a few tokens (from 9 rows on, and the thin GEMM from 3).
 
 The HIP GEMM runs through the C ABI (nn_amd -> libnnq.so) and is compared with the
 CPU oracle on the same bytes and activations (tolerances as in test_gpu_linear):

@@ -1,4 +1,5 @@
-"""GPU parity for the Q8_0 / Q6_K prefill GEMM (m > 8 tokens, nnq_gemm_blk.hip).
+"""GPU parity for the Q8_0 / Q6_K prefill GEMM (nnq_gemm_blk.hip) and the kernels beside it (up to 16
+rows nnq_gemm_few.hip, over 128 bf16 rows nnq_gemm_wide8.hip and nnq_gemm_wide6.hip).
 
 QLinear::forward with a batch of tokens over these formats
 (crates/nn-core/src/layers/quantized/linear.rs:366-400, quantized_matmul_core,
@@ -11,9 +12,9 @@ error <= 1e-3, per-row cosine >= 0.99999):
   * quantized N(0, 0.02) weights at the Qwen3-8B / GPT-OSS shapes;
   * Q8_0 rows whose block count is padded to groups of 8 (K = 2880, 4128);
   * f32 (hi + lo staging) and bf16 activations, f32 and bf16 outputs, bias, row counts
-    that leave partial tiles (m = 9, 33, 130, 320 and 1100: the 128-row and, with bf16
-    input, 128-column tiles; n = 96 and 520 leave a partial column tile), and m = 8 /
-    m = 9 consistency (GEMV vs GEMM).
+    that leave partial tiles (m = 9 in the few-row kernel; 33, 130, 320 and 1100: the 128-row
+    and, with bf16 input, 128-column tiles; n = 96 and 520 leave a partial column tile), and
+    m = 8 / m = 9 consistency.
 """
 import numpy as np
 import pytest
@@ -177,12 +178,16 @@ def test_gemm_q80_wide(O, dev, m, n, k):
 
 # The wide Q6_K kernel (bf16 x, more than 128 rows, whole groups of 8 weight tiles): one row past
 # its lower limit, ragged row tiles, K not split and split 2, 3, 4, 7 and 8 ways, the fewest
-# super-blocks of a part, every sign of the int8 scales (and one shape it leaves to the block kernel).  Bar: products are exact in f32, so max |error| <= 1e-5 of
-# the output's rms (f32 sums over K <= 12288; 9e-7 measured at 512 x 4096 x 12288).
-@pytest.mark.parametrize("m,n,k", [(129, 24576, 512), (385, 8192, 1536), (200, 8192, 1536), (300, 4096, 2048),
-                                   (517, 1536, 3584), (200, 4096, 6144), (512, 12288, 512), (1025, 4096, 1536)])
-def test_wide_q6k(m, n, k):
+# super-blocks of a part, every sign of the int8 scales (and one shape that the rule leaves to the
+# block kernel: split 0).  Bar: products are exact in f32, so max |error| <= 1e-5 of the output's
+# rms (f32 sums over K <= 12288; 9e-7 measured at 512 x 4096 x 12288).
+@pytest.mark.parametrize("m,n,k,split", [(129, 24576, 512, 1), (385, 8192, 1536, 2),
+                                         (200, 8192, 1536, 3), (300, 4096, 2048, 4), (517, 1536, 3584, 7),
+                                         (129, 4096, 4096, 8), (200, 4096, 6144, 8), (512, 12288, 512, 1),
+                                         (1025, 4096, 1536, 0)])
+def test_wide_q6k(rules, m, n, k, split):
     import nn_amd
+    assert rules.wide6(m, n, k) == split
     nn_amd.init(0)
     b = nn_amd.quantize_q6_k(nn_amd.synth_normal(m, 1, (n, k), 0.02)).reshape(-1, 210).copy()
     b[::3, 192:208] = (256 - b[::3, 192:208].astype(np.int32)).astype(np.uint8)  # negated scales

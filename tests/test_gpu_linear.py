@@ -206,10 +206,9 @@ def test_q4k_decode_launch_shapes(O, dev, k, m, xdt):
                                        ("q8_0", 12, "f32"), ("q8_0", 16, "f32"), ("q8_0", 17, "f32"), ("q8_0", 5, "bf16"),
                                        ("q6_k", 3, "bf16"), ("q6_k", 9, "bf16"), ("q6_k", 5, "f32")])
 def test_linear_gemm_crossover(O, dev, fmt, m, xdt):
-    """Batches on both sides of each format's GEMV-to-GEMM crossover (Q4_K from 3 tokens
-    with bf16 activations and from 9 with f32 ones, Q6_K from 9, Q8_0 from 9 with bf16
-    and from 17 with f32 ones; smaller Q8_0 and Q6_K batches run the batched decode
-    kernels in passes of 8 and 4 tokens), with a ragged tile."""
+    """Batches on both sides of each format's line between decode GEMV passes (of up to 4 tokens)
+    and the GEMMs: Q4_K from 3 tokens with bf16 activations (the thin GEMM) and from 7 with
+    f32 ones, Q8_0 and Q6_K from 5 (the few-row GEMM up to 16 tokens), with a ragged tile."""
     import nn_amd
     n, k = 200, 1024
     b = quantized_weight_bytes(fmt, n, k, seed=300 + m, O=O)

@@ -2,8 +2,8 @@
 
 nn_amd.QuantizedMLP runs through the C ABI (nnq_mlp_forward): for m <= 2 the gate | up
 GEMV and a down GEMV that forms silu(gate) * up while staging its input; for larger m
-the gate | up linear (GEMM for Q4_K beyond 8 tokens), a SwiGLU kernel and the down
-linear.  The oracle composes the reference's steps on the same block bytes
+the gate | up linear, a SwiGLU kernel and the down linear (the wide prefill GEMM of an
+interleaved Q4_K gate | up includes the SwiGLU).  The oracle composes the reference's steps on the same block bytes
 (QLinear::forward / quantized_matmul per format, silu, product, down).  Bars as in
 test_gpu_linear: normwise and elementwise max relative error <= 1e-3 (near-zero skip
 at 1% of the peak), per-row cosine >= 0.99999; bf16 outputs equal the f32 result
