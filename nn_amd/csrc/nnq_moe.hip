@@ -847,14 +847,23 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
             }
             // Every step issues the same batch on every wave: the weights of chunk t + PF
             // (clamped into range; idle waves load block 0), then the copies of chunk
-            // t + NBUF - 1.  The prologue runs steps t = 1 - NBUF .. -1 the same way, so
-            // before chunk ch is read exactly NBUF - 2 batches follow its copies.
-            auto step = [&](int t, int wslot) {
-                wload(max(t + PF, 0), wslot);
+            // t + NBUF - 1.  The prologue issues the batches of steps t = 1 - NBUF .. -1, all
+            // their copies before all their loads (and the compiler may not mix them), so
+            // before chunk ch is read at most NBUF - 2 batches follow its copies.  The steps
+            // of the last chunks (TAIL) load no weights: nothing would use
+            // them, so the compiler deletes such loads, and a wait that counted them would
+            // not cover the chunk's copies.  Their waits count copies only, which is right
+            // whatever else is in flight.
+            auto step = [&](int t, int wslot, auto tail_c) {
+                if constexpr (!decltype(tail_c)::value) wload(max(t + PF, 0), wslot);
                 issue(t + NBUF - 1);
             };
 #pragma unroll
-            for (int t = 1 - NBUF; t < 0; t++) step(t, ((t + PF) % (PF + 1) + (PF + 1)) % (PF + 1));
+            for (int t = 1 - NBUF; t < 0; t++) issue(t + NBUF - 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 1 - NBUF; t < 0; t++) wload(max(t + PF, 0), ((t + PF) % (PF + 1) + (PF + 1)) % (PF + 1));
+            __builtin_amdgcn_sched_barrier(0);
             // lane holds rows 4p + i of each tile; acc[.][.][0]: column 2 * l16 of the block,
             // [1]: 2 * l16 + 1
             auto epilogue = [&](auto &acc) {
@@ -922,12 +931,13 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
                 for (int b = 0; b < NBW; b++)
 #pragma unroll
                     for (int mt = 0; mt < MTN; mt++) acc[b][mt][0] = acc[b][mt][1] = zero4();
-                auto body = [&](int ch, int slot) {
-                    wait_vmcnt<(NBUF - 2) * (LPA + WPS)>();  // this thread's copies of chunk ch
+                auto body = [&](int ch, int slot, auto tail_c) {
+                    constexpr bool TAIL = decltype(tail_c)::value;
+                    wait_vmcnt<(NBUF - 2) * (TAIL ? LPA : LPA + WPS)>();  // this thread's copies of chunk ch
                     __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0): this wave's reads of chunk ch - 1
                     __builtin_amdgcn_s_barrier();            // everyone's copies of chunk ch have landed
                     __builtin_amdgcn_sched_barrier(0);
-                    step(ch, (slot + PF) % (PF + 1));
+                    step(ch, (slot + PF) % (PF + 1), tail_c);
                     if (!active) return;
                     const unsigned char *buf = smem + (size_t)(ch % NBUF) * C::BUF;
 #pragma unroll
@@ -972,11 +982,11 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_stream_kernel(MoeDev d, Mo
                 const int nfull = nch - nch % (PF + 1);
                 for (int c0 = 0; c0 < nfull; c0 += PF + 1) {
 #pragma unroll
-                    for (int u = 0; u < PF + 1; u++) body(c0 + u, u);
+                    for (int u = 0; u < PF + 1; u++) body(c0 + u, u, std::false_type{});
                 }
 #pragma unroll
                 for (int u = 0; u < PF; u++)
-                    if (nfull + u < nch) body(nfull + u, u);
+                    if (nfull + u < nch) body(nfull + u, u, std::true_type{});
                 __builtin_amdgcn_s_waitcnt(0);  // trailing copies and weight loads (unused)
                 if (!active) return;
                 epilogue(acc);
