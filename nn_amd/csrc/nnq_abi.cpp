@@ -501,12 +501,15 @@ static bool gemm_batch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
 // first launch's rows, or the last, shorter one's when that plan needs more).  y is the output
 // the launches get (null: any 16-byte aligned one): the wide kernels take only such outputs, and
 // the block kernel that runs in their place has other scratch.  (A later launch's y is as
-// aligned as the first's: those kernels' rows are whole 16-column tiles.)
-static size_t gemm_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype, const void *y) {
+// aligned as the first's: those kernels' rows are whole 16-column tiles.)  swiglu_out: the launch
+// that writes h (prefill_swiglu), whose plan is its own.
+static size_t gemm_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype, const void *y, int swiglu_out = 0) {
     const int64_t mc = gemm_chunk_rows(m, w->L.k), tail = m % mc;
-    void *yp = const_cast<void *>(y);
-    size_t b = gemm_scratch_bytes(gemm_args(w, nullptr, x_dtype, mc, nullptr, yp, NNQ_F32));
-    if (tail) b = std::max(b, gemm_scratch_bytes(gemm_args(w, nullptr, x_dtype, tail, nullptr, yp, NNQ_F32)));
+    GemmArgs g = gemm_args(w, nullptr, x_dtype, mc, nullptr, const_cast<void *>(y), NNQ_F32);
+    g.swiglu_out = swiglu_out;
+    size_t b = gemm_scratch_bytes(g);
+    g.m = tail;
+    if (tail) b = std::max(b, gemm_scratch_bytes(g));
     return b;
 }
 
@@ -516,17 +519,20 @@ static size_t few_call_scratch(const nnq_weight *w, int64_t m, nnq_dtype x_dtype
     return gemm_few_scratch_bytes(gemm_args(w, nullptr, x_dtype, rows, nullptr, nullptr, NNQ_F32), w->L.fmt);
 }
 
-static size_t linear_scratch_bytes(const nnq_weight *w, int64_t m, nnq_dtype x_dtype, const void *y) {
+static size_t linear_scratch_bytes(const nnq_weight *w, int64_t m, nnq_dtype x_dtype, const void *y,
+                                   int swiglu_out = 0) {
     if (few_batch(w, m, x_dtype)) return few_call_scratch(w, m, x_dtype);
     if (!gemm_batch(w, m, x_dtype)) return 0;
-    return gemm_call_scratch(w, m, x_dtype, y);
+    return gemm_call_scratch(w, m, x_dtype, y, swiglu_out);
 }
 
 // whether a prefill of m tokens can write h = silu(gate) * up from the gate | up GEMM: Q4_K, one
 // launch (the rows of y differ from the chunks' otherwise), the wide kernel without a K split
 static bool prefill_swiglu(const nnq_weight *w, int64_t m, nnq_dtype x_dtype) {
-    return w->L.fmt == NNQ_FMT_Q4_K && m > 2 && gemm_batch(w, m, x_dtype) && gemm_chunk_rows(m, w->L.k) == m &&
-           gemm_wide_swiglu(gemm_args(w, nullptr, x_dtype, m, nullptr, nullptr, NNQ_F32));
+    if (w->L.fmt != NNQ_FMT_Q4_K || m <= 2 || !gemm_batch(w, m, x_dtype) || gemm_chunk_rows(m, w->L.k) != m) return false;
+    GemmArgs g = gemm_args(w, nullptr, x_dtype, m, nullptr, nullptr, NNQ_F32);
+    g.swiglu_out = 1;
+    return gemm_wide_swiglu(g);
 }
 
 static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype, int64_t m, const float *bias,
@@ -549,7 +555,7 @@ static int dispatch_linear(const nnq_weight *w, const void *x, nnq_dtype x_dtype
         Scratch s;
         void *scr = ext_scratch;
         if (!scr) {
-            HIP_TRY(s.alloc(gemm_call_scratch(w, m, x_dtype, y), (hipStream_t)stream), "scratch alloc");
+            HIP_TRY(s.alloc(gemm_call_scratch(w, m, x_dtype, y, swiglu_out), (hipStream_t)stream), "scratch alloc");
             scr = s.p;
         }
         for (int64_t m0 = 0; m0 < m; m0 += mc) {
@@ -969,7 +975,7 @@ int nnq_mlp_forward(const nnq_mlp *p, const void *x, nnq_dtype x_dtype, int64_t 
         return size_fail();
     const bool xm = misaligned_in(x), ym = misaligned_out(y);
     const size_t lin_bytes =
-        std::max(linear_scratch_bytes(p->gu, m, x_dtype, nullptr),
+        std::max(linear_scratch_bytes(p->gu, m, x_dtype, nullptr, hout ? 1 : 0),
                  fused ? 0 : linear_scratch_bytes(p->down, m, NNQ_F32, ym ? nullptr : y));
     const size_t sizes[5] = {gu_bytes, h_bytes, lin_bytes, xm ? xbytes : 0, ym ? ybytes : 0};
     size_t off[5], total = 0;

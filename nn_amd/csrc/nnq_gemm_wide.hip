@@ -695,10 +695,10 @@ __global__ __launch_bounds__(512) void gemm_stage_wide_kernel(const void *xv, in
 // output (the epilogue writes 16-byte row chunks).
 int gemm_wide_plan(const GemmArgs &a, int *ks) {
     if (a.blk || a.n != a.ntile * 16 || (reinterpret_cast<uintptr_t>(a.y) & 15)) return 0;
-    return nnq_rule_gemm_wide(a.m, a.ntile, a.nblk, a.x_bf16, ks);
+    return nnq_rule_gemm_wide(a.m, a.ntile, a.nblk, a.x_bf16, a.swiglu_out, ks);
 }
 
-// whether the call can write silu(gate) * up (swiglu_out) from the wide kernel's epilogue
+// whether the call (a.swiglu_out set) can write silu(gate) * up from the wide kernel's epilogue
 bool gemm_wide_swiglu(const GemmArgs &a) {
     int ks = 0;
     return gemm_wide_plan(a, &ks) && ks == 1;

@@ -81,7 +81,7 @@ constexpr int kMoeFewAssign = 128;  //   and assignments (two per lane of its ba
 extern "C" {
 int nnq_rule_few_rows(int fmt, int64_t ntile, int64_t k, int64_t m, int x_bf16);  // 1: gemm_few_kernel
 int nnq_rule_gemm_ring(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *bn, int *bm);
-int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *ks);
+int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int h_out, int *ks);
 int nnq_rule_gemm_wide6(int64_t m, int64_t ntile, int64_t nblk);
 int nnq_rule_moe_few(int64_t experts, int64_t hidden, int64_t inter, int64_t tokens, int top_k, int x_bf16);
 }

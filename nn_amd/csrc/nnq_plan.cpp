@@ -139,8 +139,11 @@ int nnq_rule_gemm_ring(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *
 // Both sides' times are estimated with constants fitted to 288 calls of the ring and 713 of this
 // kernel, 4% and 5% off in the mean: us, per million of x, per MB of slabs (the ring's two planes have
 // one each), per round and per super-block of a round (the ring's 128-column tiles 0.8 of its wide ones).
+// h_out: the call is an MLP's gate | up and wants h = silu(gate) * up, which this kernel writes itself
+// where K is not split and the ring leaves to a launch of about 4 us (f32 forwards, ring / wide gate | up: 260
+// tokens of 768 x 2048 49.5 / 44.4 us, 129 of 1792 x 4608 66.3 / 61.7; 129 of 2816 x 4096 72.0 / 78.8).
 // Returns the column tiles per workgroup (0: the ring kernel takes the shape) and the K split.
-int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *ks) {
+int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int h_out, int *ks) {
     if (m <= 128 || nblk > 48) return 0;
     const int64_t nrt = (m + 255) / 256, n = ntile * 16;
     const int tiles[3] = {6, 4, 8};
@@ -175,7 +178,7 @@ int nnq_rule_gemm_wide(int64_t m, int64_t ntile, int64_t nblk, int x_bf16, int *
         const float wide = 7.1f + 1.37f * x_m + (float)rounds * (3.8f + (float)(nblk / best_ks) * f32_us[at]) + slabs;
         const float ring = 10.4f + 1.05f * x_m + 0.34f * (float)(2 * rks + 1) * y_mb +
                            3.15f * (float)(rrounds * (nblk / rks)) * (bn == 192 ? 1.0f : 0.8f);
-        if (ring < wide) return 0;
+        if (ring + (h_out && best_ks == 1 ? 4.0f : 0.0f) < wide) return 0;
     }
     if (ks) *ks = best_ks;
     return tiles[at];

@@ -38,7 +38,7 @@ def rules():
     lib = _lib.load()
     i64, c_int = ctypes.c_int64, ctypes.c_int
     lib.nnq_rule_few_rows.argtypes = [c_int, i64, i64, i64, c_int]
-    lib.nnq_rule_gemm_wide.argtypes = [i64, i64, i64, c_int, ctypes.POINTER(c_int)]
+    lib.nnq_rule_gemm_wide.argtypes = [i64, i64, i64, c_int, c_int, ctypes.POINTER(c_int)]
     lib.nnq_rule_gemm_wide6.argtypes = [i64, i64, i64]
     lib.nnq_rule_moe_few.argtypes = [i64, i64, i64, i64, c_int, c_int]
 
@@ -48,10 +48,10 @@ def rules():
             return lib.nnq_rule_few_rows(fmt, (n + 15) // 16, k, m, bf16)
 
         @staticmethod
-        def wide(m, n, k, bf16):
+        def wide(m, n, k, bf16, h_out=0):
             """(column tiles per workgroup, K split); (0, 0) where the wide Q4_K kernel does not take it"""
             ks = c_int(0)
-            return lib.nnq_rule_gemm_wide(m, n // 16, k // 256, bf16, ctypes.byref(ks)), ks.value
+            return lib.nnq_rule_gemm_wide(m, n // 16, k // 256, bf16, h_out, ctypes.byref(ks)), ks.value
 
         @staticmethod
         def wide6(m, n, k):

@@ -118,3 +118,19 @@ def test_wide6_where_it_is_faster(rules, m, n, k, wide):
 ])
 def test_wide_tiles_where_they_are_faster(rules, m, n, k, bf16, tiles, split):
     assert rules.wide(m, n, k, bf16) == (tiles, split)
+
+
+# f32 prefill MLPs measured with either kernel under their gate | up (us, ring kernel and SwiGLU launch / wide kernel).
+@pytest.mark.parametrize("m,hidden,inter,wide", [
+    (260, 768, 2048, 4),    # 49.5 / 44.3
+    (260, 1024, 2560, 4),   # 49.9 / 47.7
+    (129, 1792, 4608, 4),   # 66.3 / 61.4
+    (260, 3328, 4864, 8),   # 151.8 / 146.5
+    (260, 1792, 2560, 0),   # 62.4 / 66.1
+    (129, 2816, 4096, 0),   # 71.5 / 78.3
+    (260, 3328, 8704, 0),   # 251.0 / 258.5
+])
+def test_wide_swiglu_where_it_is_faster(rules, m, hidden, inter, wide):
+    """The launch that the ring kernel's MLP has more is counted, in calls that can write h themselves only."""
+    assert rules.wide(m, 2 * inter, hidden, 0, 1)[0] == wide
+    assert rules.wide(m, 2 * inter, hidden, 0) == (0, 0)
